@@ -846,78 +846,137 @@ __global__ __launch_bounds__(NT, WG_PER_CU) void ns_px_bf16(NsArgs a, int total)
 }
 
 // ---------------------------------------------------------------------------
-// fp32 Newton-Schulz (the pretrain copy keeps the buffer dtype) on the fp32
-// matrix cores (v_mfma_f32_32x32x2_f32, fp32 products and accumulation).
-// 128 x 128 output tiles per 256-thread workgroup, 4 waves of 64 x 64 (2 x 2
-// MFMA tiles of 32 x 32, 32 MFMAs per wave and K tile); K advances 16 per
-// tile, double-buffered in LDS: the next tile's global loads (into registers)
-// are in flight during the current tile's MFMAs and stored to the other buffer
-// after them.  Operands reach LDS in one of two forms:
-//   RK: operand rows, [row][k] (rows of X for SYRK; rows of A / P, and by
-//       symmetry A's columns), 17 floats per row, so the 32 lanes that read
-//       one k of 32 consecutive rows hit 32 different banks;
-//   KC: [k][col] (PX's X operand, k = rows of X), 132 floats per row, 16-B
-//       aligned for float4 stores.
+// fp32 Newton-Schulz (the pretrain copy keeps the buffer dtype) on the bf16
+// matrix cores.  An fp32 value is the exact sum of three bf16 values
+// (h = bf16(x), m = bf16(x - h), l = x - h - m: 8 + 8 + 8 significant bits, signs
+// included), and a product of two of them is taken as the six terms
+//   hh + hm + mh + hl + lh + mm
+// (Henry, Tang, Heinecke: Leveraging the bfloat16 artificial intelligence datatype
+// for higher-precision computations, 2019), accumulated in fp32 by
+// v_mfma_f32_32x32x16_bf16.  The dropped ml, lm and ll are below 2^-23 of the
+// product's leading term and of random sign, and the accumulators are rounded once
+// per 16 terms instead of once per two (v_mfma_f32_32x32x2_f32): against fp64 the
+// five iterations are off by 0.6-1.2e-6 on Gaussian blocks from 96 x 136 to
+// 1024 x 2752, where the fp32 MFMA gave 1.4-3.4e-6, and by 3.0-5.0e-6 against
+// 6.9-13.6e-6 on singular values spread over four decades.
+//
+// Why: six such MFMAs take 192 cycles for 16 k against 512 of the fp32 MFMA, which
+// bound these kernels (71% busy at the 1.3B shapes).  Measured there, 176 blocks of
+// 512 x 512: SYRK 297 -> 168 us, POLY 302 -> 181, PX 407 -> 265, PX + apply 469 ->
+// 322; 48 of 512 x 1376: SYRK 198 -> 118.  Now no unit is full: the MFMAs are busy
+// 46-53% of the cycles at 1.8-1.9 GHz (the package-power limit), the LDS reads and
+// writes of a step take 0.75 of its MFMA time and the split's VALU work 0.55.
+// Measured without gain: the split's subtractions as v_dot2_f32_bf16 (slower),
+// raised wave priority during the MFMAs, the lower-left wave of a diagonal tile
+// left idle, one accumulator and three waves per SIMD (SYRK 190 us, and see lo).
+//
+// Tiles of FT x FT (FT = 64 TW) per 256-thread workgroup, 2 x 2 waves of TW x TW
+// MFMA tiles; K advances 16 per step, double-buffered in LDS: the next step's
+// global loads (fp32, into registers) are in flight during the current step's
+// MFMAs, are split after them and stored to the other buffer as three bf16 planes.
+// Operands reach LDS in one of two forms, 16 k x FT x 2 B per plane:
+//   K: operand rows, [row][16 k] (rows of X for SYRK; rows of A / P, and by
+//      symmetry A's columns).  A row is two 16-B chunks; chunk c of row r sits at
+//      c ^ ((r >> 3) & 1), so the 16 rows of a quarter-wave's ds_read_b128 cover
+//      all 64 banks;
+//   T: [k][FT columns] (PX's X operand, k = rows of X), read with
+//      ds_read_b64_tr_b16; the 64-B chunk of columns 32 p .. 32 p + 31 of row k sits
+//      at p ^ (k & 3) (FT = 128) or p ^ ((k >> 1) & 1) (FT = 64), so the four rows
+//      of a transposed read lie in different banks.
 // SYRK and POLY produce symmetric matrices: only the tiles on and above the
 // diagonal are computed, each stored with its mirror (staged in LDS so both
-// stores are row-contiguous), so the stored matrix is exactly symmetric.
+// stores are row-contiguous), so the stored matrix is exactly symmetric.  A tile
+// that lies in the zero padding is stored as zeros without running its products.
 // ---------------------------------------------------------------------------
-constexpr int FT = 128;                // output tile
-constexpr int FK = 16;                 // K tile
 constexpr int F_NT = 256;              // 4 waves, 2 x 2
-constexpr int RK_LD = FK + 1;
-constexpr int KC_LD = FT + 4;
-constexpr int F_OPER = FT * RK_LD;     // floats per operand buffer
-static_assert(FK * KC_LD <= F_OPER, "both forms fit one operand buffer");
-constexpr int F_ST = FT + 1;           // staged tile: 129 floats per row
-constexpr int F_HALF = FT / 2;         // the tile is staged and stored half its rows at a time
-static_assert(F_HALF * F_ST <= 4 * F_OPER, "half the staged tile fits in the operand buffers");
-constexpr int F_APPLY_BATCH = 8;       // parameter elements per batch of the apply's loads
-constexpr int F_RQ = FK / 4;           // float4 per operand row of a K tile
-constexpr int F_QPT = FT * FK / 4 / F_NT;  // float4 per thread and operand K tile
+constexpr int FK = 16;                 // K per step
+constexpr int F_PAD = 128;             // padding granularity of the fp32 stacks
+// Tiles of 128 x 128 from which a launch uses them, about one per CU; with fewer,
+// 64 x 64 tiles spread the work over more CUs (measured: 48 blocks of 512 x 1376,
+// 480 tiles: SYRK 139 us with 64 x 64 tiles, 118 with 128 x 128; 44 blocks of 256 x
+// 256, 132 tiles: 12.4 against 16.3; 12 blocks of 256 x 688, 36 tiles: 16.1 against 29.7).
+constexpr int F32_FILL = 256;
 
-// One operand's K tile in registers.
-struct F32Stage {
-  float4 v[F_QPT];
+template <int TW>
+struct F32Geo {
+  static constexpr int FT = 64 * TW;              // output tile
+  static constexpr int WT = 32 * TW;              // wave sub-tile
+  static constexpr int PLANE = FT * FK * 2;       // bytes of one bf16 plane of an operand's K step
+  static constexpr int OPER = 3 * PLANE;          // bytes of an operand's K step
+  static constexpr int QPT = FT * FK / 4 / F_NT;  // float4 per thread and operand K step
+  static constexpr int LDS = 4 * OPER;            // [buffer 0: A, B][buffer 1: A, B]
+  static_assert(64 * FT * 4 <= LDS, "64 rows of the staged tile fit in the operand buffers");
+  static_assert(QPT == TW, "whole float4 loads per thread");
 };
 
-// rows r0 .. r0+127 of a row-major matrix (leading dimension ld), k0 .. k0+FK-1
-__device__ __forceinline__ void f32_load_rows(F32Stage& g, const float* src, int64_t ld, int r0, int k0) {
-#pragma unroll
-  for (int j = 0; j < F_QPT; ++j) {
-    const int idx = threadIdx.x + F_NT * j;
-    g.v[j] = *reinterpret_cast<const float4*>(src + int64_t(r0 + idx / F_RQ) * ld + k0 + 4 * (idx % F_RQ));
-  }
+// This thread's float4 j of an operand's K step: rows r0 .. r0+FT-1, k0 .. k0+FK-1 of
+// a row-major matrix (leading dimension ld) ...
+template <int TW>
+__device__ __forceinline__ const float* f32_src_rows(const float* src, int64_t ld, int r0, int j) {
+  const int idx = threadIdx.x + F_NT * j;
+  return src + int64_t(r0 + (idx >> 2)) * ld + 4 * (idx & 3);
 }
-__device__ __forceinline__ void f32_store_rk(const F32Stage& g, float* s) {
-#pragma unroll
-  for (int j = 0; j < F_QPT; ++j) {
-    const int idx = threadIdx.x + F_NT * j;
-    float* d = s + (idx / F_RQ) * RK_LD + 4 * (idx % F_RQ);
-    d[0] = g.v[j].x;
-    d[1] = g.v[j].y;
-    d[2] = g.v[j].z;
-    d[3] = g.v[j].w;
-  }
+// ... or rows k0 .. k0+FK-1 of X (leading dimension ld), columns c0 .. c0+FT-1
+template <int TW>
+__device__ __forceinline__ const float* f32_src_cols(const float* X, int64_t ld, int c0, int j) {
+  constexpr int Q = F32Geo<TW>::FT / 4;
+  const int idx = threadIdx.x + F_NT * j;
+  return X + int64_t(idx / Q) * ld + c0 + 4 * (idx % Q);
 }
-// rows k0 .. k0+FK-1 of X (leading dimension ld), columns c0 .. c0+127
-__device__ __forceinline__ void f32_load_kc(F32Stage& g, const float* X, int64_t ld, int c0, int k0) {
-#pragma unroll
-  for (int j = 0; j < F_QPT; ++j) {
-    const int idx = threadIdx.x + F_NT * j;
-    g.v[j] = *reinterpret_cast<const float4*>(X + int64_t(k0 + (idx >> 5)) * ld + c0 + 4 * (idx & 31));
+
+// Splitting four values into three planes of four bf16 values each, PLANE bytes
+// apart from d, in six parts of two to six VALU instructions, so that the main
+// loop can put one part behind each of its MFMAs.
+struct F32Split {
+  uint32_t h0, h1, m0, m1;
+  float a0, a1, a2, a3;
+  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+  template <int PLANE>
+  __device__ __forceinline__ void part(int n, const float4& v, char* d) {
+    switch (n) {
+      case 0:
+        h0 = f2bf2(v.x, v.y);
+        h1 = f2bf2(v.z, v.w);
+        break;
+      case 1:
+        a0 = v.x - lo(h0);
+        a1 = v.y - hi(h0);
+        break;
+      case 2:
+        a2 = v.z - lo(h1);
+        a3 = v.w - hi(h1);
+        *reinterpret_cast<uint2*>(d) = make_uint2(h0, h1);
+        break;
+      case 3:
+        m0 = f2bf2(a0, a1);
+        m1 = f2bf2(a2, a3);
+        *reinterpret_cast<uint2*>(d + PLANE) = make_uint2(m0, m1);
+        break;
+      case 4:
+        a0 -= lo(m0);
+        a1 -= hi(m0);
+        a2 -= lo(m1);
+        break;
+      default:
+        a3 -= hi(m1);
+        *reinterpret_cast<uint2*>(d + 2 * PLANE) = make_uint2(f2bf2(a0, a1), f2bf2(a2, a3));
+    }
   }
+};
+// LDS offset, within an operand's buffer, of this thread's float4 j
+template <int TW>
+__device__ __forceinline__ uint32_t f32_off_k(int j) {
+  const int idx = threadIdx.x + F_NT * j, r = idx >> 2, q = idx & 3;
+  return uint32_t(r * 32 + (((q >> 1) ^ ((r >> 3) & 1)) << 4) + ((q & 1) << 3));
 }
-__device__ __forceinline__ void f32_store_kc(const F32Stage& g, float* s) {
-  // a native 4-wide vector store (a float4 struct copy here kept the staged
-  // tile in scratch memory)
-  typedef float f32x4_t __attribute__((ext_vector_type(4)));
-#pragma unroll
-  for (int j = 0; j < F_QPT; ++j) {
-    const int idx = threadIdx.x + F_NT * j;
-    const f32x4_t v = {g.v[j].x, g.v[j].y, g.v[j].z, g.v[j].w};
-    *reinterpret_cast<f32x4_t*>(s + (idx >> 5) * KC_LD + 4 * (idx & 31)) = v;
-  }
+template <int TW>
+__device__ __forceinline__ int f32_tswz(int k) { return TW == 2 ? (k & 3) : ((k >> 1) & 1); }
+template <int TW>
+__device__ __forceinline__ uint32_t f32_off_t(int j) {
+  constexpr int FT = F32Geo<TW>::FT, Q = FT / 4;
+  const int idx = threadIdx.x + F_NT * j, k = idx / Q, n = 4 * (idx % Q);
+  return uint32_t(k * FT * 2 + (((n >> 5) ^ f32_tswz<TW>(k)) << 6) + ((n & 31) << 1));
 }
 
 // Upper tile t of an nt x nt grid of tiles (ti <= tj), row-major over the
@@ -932,188 +991,355 @@ __device__ __forceinline__ void f32_sym_tile(int t, int nt, int& ti, int& tj) {
   tj = i + t;
 }
 
-// Add v to the diagonal entries of an RK-form K tile in registers: rows rbase
-// + 0..127 of the operand, k0 .. k0+FK-1; an element is on the diagonal when
-// its row equals its k.  The quintic's linear terms enter the products this
-// way: PX multiplies (P + a I) X, POLY A (A + (b/c) I); no epilogue reads
-// global memory and no accumulator leaves the matrix registers.
-__device__ __forceinline__ void f32_add_diag(F32Stage& g, int rbase, int k0, float v) {
+// Swizzle of the staged output tile's 16-B chunks within a column: distinct for 16
+// consecutive columns (the accumulator writes) and for 16 columns four apart (the
+// 4 x 4 block reads).
+__device__ __forceinline__ int f32_tile_swz(int c) { return ((c >> 2) & 15) ^ ((c & 3) << 2); }
+
+// param[pr][pc .. pc+3] += alpha s v[k] over this thread's N chunks (at(k, pr, pc)
+// gives chunk k's place), one rounding to the parameter dtype per element, as
+// torch's foreach add with alpha.  All loads are issued before the first store.
+// rows, cols: the parameter block's sides.
+template <class TP, int N, class At>
+__device__ __forceinline__ void f32_update(typename TP::storage* prm, const NsArgs& a, float s, const float4 (&v)[N],
+                                           At&& at, int rows, int cols) {
+  const bool vec = a.vec && cols % 4 == 0;  // 16-B (bf16: 8-B) accesses
+  float p[N][4];
 #pragma unroll
-  for (int j = 0; j < F_QPT; ++j) {
-    const int idx = threadIdx.x + F_NT * j;
-    const int d = rbase + idx / F_RQ - (k0 + 4 * (idx % F_RQ));  // row - k of the float4's first element
-    if (d == 0) g.v[j].x += v;
-    if (d == 1) g.v[j].y += v;
-    if (d == 2) g.v[j].z += v;
-    if (d == 3) g.v[j].w += v;
+  for (int k = 0; k < N; ++k) {
+    int pr, pc;
+    at(k, pr, pc);
+    const int64_t o = int64_t(pr) * cols + pc;
+    if (vec && pr < rows && pc < cols) {
+      if constexpr (sizeof(typename TP::storage) == 2) {
+        const uint2 w = *reinterpret_cast<const uint2*>(prm + o);
+        p[k][0] = __uint_as_float(w.x << 16);
+        p[k][1] = __uint_as_float(w.x & 0xffff0000u);
+        p[k][2] = __uint_as_float(w.y << 16);
+        p[k][3] = __uint_as_float(w.y & 0xffff0000u);
+      } else {
+        const float4 w = *reinterpret_cast<const float4*>(prm + o);
+        p[k][0] = w.x;
+        p[k][1] = w.y;
+        p[k][2] = w.z;
+        p[k][3] = w.w;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[k][e] = pr < rows && pc + e < cols ? TP::load(prm, o + e) : 0.f;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    int pr, pc;
+    at(k, pr, pc);
+    const int64_t o = int64_t(pr) * cols + pc;
+    const float u[4] = {s * v[k].x, s * v[k].y, s * v[k].z, s * v[k].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[k][e] = fmaf(a.alpha, u[e], p[k][e]);
+    if (vec && pr < rows && pc < cols) {
+      if constexpr (sizeof(typename TP::storage) == 2)
+        *reinterpret_cast<uint2*>(prm + o) = make_uint2(f2bf2(p[k][0], p[k][1]), f2bf2(p[k][2], p[k][3]));
+      else
+        *reinterpret_cast<float4*>(prm + o) = make_float4(p[k][0], p[k][1], p[k][2], p[k][3]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (pr < rows && pc + e < cols) TP::store(prm, o + e, p[k][e]);
+    }
   }
 }
 
-// 16-deep K tiles double-buffered in 35 KiB of LDS, so four workgroups share a
-// CU (three for the apply, whose epilogue holds more registers; at least three
-// waves per SIMD, which hide each other's barrier and load waits: one
-// workgroup per CU measured 18% slower than two, four 3% faster than two).
-// The 128 x 128 output tile is staged and stored in two halves of 64 rows (the
-// rows of one wave row, wr), each in the operand buffers.
-template <int STAGE, class TP>
-__global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(3))) void ns_f32(NsArgs a) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * F_OPER];  // [buffer 0: A, B][buffer 1: A, B]
+template <int STAGE, class TP, int TW>
+__global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(2))) void ns_f32(NsArgs a) {
+  using G = F32Geo<TW>;
+  constexpr int FT = G::FT, WT = G::WT;
+  __shared__ __attribute__((aligned(1024))) char lds[G::LDS];
   constexpr bool PX = STAGE == NS_PX || STAGE == NS_PX_APPLY;
   constexpr bool SYM = STAGE == NS_SYRK || STAGE == NS_POLY;
-  const int b = blockIdx.y;
+  const int nt = a.mp / FT, nc = a.np / FT;
+  const int tiles = SYM ? nt * (nt + 1) / 2 : nt * nc;
+  int b, t0;
+  if (!decode_tile(blockIdx.x, tiles, a.N, b, t0)) return;
   int ti, tj;
   if (SYM) {
-    f32_sym_tile(blockIdx.x, a.mp / FT, ti, tj);
+    f32_sym_tile(t0, nt, ti, tj);
   } else {
-    const int nc = a.np / FT;
-    ti = blockIdx.x / nc;
-    tj = blockIdx.x % nc;
+    ti = t0 % nt;  // the tiles that read one column band of X are neighbours
+    tj = t0 / nt;
   }
   const int r0 = ti * FT, c0 = tj * FT;
   const float* X = static_cast<const float*>(a.x_in) + int64_t(b) * a.mp * a.np;
   const float* A = static_cast<const float*>(a.a_in) + int64_t(b) * a.mp * a.mp;
   const float* rsrc = STAGE == NS_SYRK ? X : A;  // rows of the row operand (and of SYRK / POLY's column operand)
   const int64_t rld = STAGE == NS_SYRK ? a.np : a.mp;
-  const int K = STAGE == NS_SYRK ? a.kx : a.mp;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wr = wave >> 1, wc = wave & 1;
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-  F32Stage ga, gb;
-  const int KT = K / FK;
-  f32_load_rows(ga, rsrc, rld, r0, 0);
-  if (PX) f32_load_kc(gb, X, a.np, c0, 0);
-  else f32_load_rows(gb, rsrc, rld, c0, 0);
-  if (PX) f32_add_diag(ga, r0, 0, a.ca);
-  if (STAGE == NS_POLY) f32_add_diag(gb, c0, 0, a.cb / a.cc);
-  f32_store_rk(ga, lds);
-  if (PX) f32_store_kc(gb, lds + F_OPER);
-  else f32_store_rk(gb, lds + F_OPER);
-  __syncthreads();
-  for (int t = 0; t < KT; ++t) {
-    const float* sa = lds + (t & 1) * 2 * F_OPER;
-    const float* sb = sa + F_OPER;
-    if (t + 1 < KT) {
-      f32_load_rows(ga, rsrc, rld, r0, (t + 1) * FK);
-      if (PX) f32_load_kc(gb, X, a.np, c0, (t + 1) * FK);
-      else f32_load_rows(gb, rsrc, rld, c0, (t + 1) * FK);
-    }
-    // 32x32x2 steps: lane l supplies row (column) l%32 at k = 2 kk + l/32
-#pragma unroll
-    for (int kk = 0; kk < FK / 2; ++kk) {
-      const int k = 2 * kk + (lane >> 5);
-      float av[2], bv[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) av[i] = sa[(wr * 64 + i * 32 + (lane & 31)) * RK_LD + k];
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        bv[j] = PX ? sb[k * KC_LD + wc * 64 + j * 32 + (lane & 31)] : sb[(wc * 64 + j * 32 + (lane & 31)) * RK_LD + k];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-    }
-    if (t + 1 < KT) {
-      float* d = lds + ((t + 1) & 1) * 2 * F_OPER;
-      if (PX) f32_add_diag(ga, r0, (t + 1) * FK, a.ca);
-      if (STAGE == NS_POLY) f32_add_diag(gb, c0, (t + 1) * FK, a.cb / a.cc);
-      f32_store_rk(ga, d);
-      if (PX) f32_store_kc(gb, d + F_OPER);
-      else f32_store_rk(gb, d + F_OPER);
-    }
-    __syncthreads();
-  }
-  const float s = a.scale != nullptr ? a.scale[b] : 1.f;
   const bool diag = SYM && tj == ti;
-  float* T = lds;  // T[r - 64 h][c]: rows 64 h .. 64 h + 63 of the tile
-  auto* prm = STAGE == NS_PX_APPLY ? reinterpret_cast<typename TP::storage*>(a.blocks[b].param) : nullptr;
-#pragma unroll 1
-  for (int h = 0; h < 2; ++h) {
-    if (h) __syncthreads();  // every wave is done reading the first half
-    // stage half h: accumulator value 4 q + e of MFMA tile (i, j) holds row
-    // 64 wr + 32 i + 8 q + 4 (lane/32) + e, column 64 wc + 32 j + lane%32, so
-    // the waves with wr == h hold the half
-    if (wr == h) {
+  // K steps over the valid extent; none where the tile holds only padding
+  const int K = STAGE == NS_SYRK ? a.kx : (a.m + FK - 1) / FK * FK;
+  const int KT = r0 >= a.m || c0 >= (PX ? a.n : a.m) ? 0 : K / FK;
+  f32x16 acc[TW][TW];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TW; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TW; ++j) acc[i][j] = f32x16{};
+  // float4 q of this thread's share of a K step: q < TW the row operand, else the
+  // column operand; dst: its LDS offset within a buffer
+  constexpr int NQ = 2 * TW;
+  const float* src[NQ];
+  uint32_t dst[NQ];
+  float4 g[2][NQ];  // K steps t + 1 and t + 2
+  const int64_t kstep_a = FK, kstep_b = PX ? int64_t(FK) * a.np : FK;
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
+  for (int j = 0; j < TW; ++j) {
+    src[j] = f32_src_rows<TW>(rsrc, rld, r0, j);
+    src[TW + j] = PX ? f32_src_cols<TW>(X, a.np, c0, j) : f32_src_rows<TW>(rsrc, rld, c0, j);
+    dst[j] = f32_off_k<TW>(j);
+    dst[TW + j] = G::OPER + (PX ? f32_off_t<TW>(j) : f32_off_k<TW>(j));
+  }
+  auto fetch = [&](float4 (&v)[NQ]) {  // the next K step
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int r = i * 32 + 8 * q + 4 * (lane >> 5) + e, c = wc * 64 + j * 32 + (lane & 31);
-              T[r * F_ST + c] = acc[i][j][4 * q + e];
-            }
+    for (int q = 0; q < NQ; ++q) {
+      v[q] = *reinterpret_cast<const float4*>(src[q]);
+      src[q] += q < TW ? kstep_a : kstep_b;
+    }
+  };
+  // per-lane fragment offsets: K form, row lane%32, k 8 (lane/32) .. +7; T form,
+  // column lane%32, the same k (two transposed reads, four k apart)
+  const int l16 = lane & 15;
+  const uint32_t kf = uint32_t((lane & 31) * 32 + (((lane >> 5) ^ ((lane >> 3) & 1)) << 4));
+  const int tk = ((lane >> 5) << 3) + (l16 >> 2);
+  const uint32_t tf = uint32_t(tk * FT * 2 + ((((lane >> 4) & 1) << 4) + ((l16 & 3) << 2)) * 2);
+  const int tz = f32_tswz<TW>(tk);
+  auto frag_k = [&](const char* s, int row, int p) {
+    return *reinterpret_cast<const bf16x8*>(s + p * G::PLANE + row * 32 + kf);
+  };
+  auto frag_t = [&](const char* s, int panel, int p) {
+    const char* q = s + p * G::PLANE + tf + ((panel ^ tz) << 6);
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(q));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(q + 4 * FT * 2));
+    typedef short i16x8 __attribute__((ext_vector_type(8)));
+    const i16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8, v);
+  };
+  F32Split sp;
+  if (KT > 0) {
+    fetch(g[0]);
+    if (KT > 1) fetch(g[1]);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int n = 0; n < 6; ++n) sp.part<G::PLANE>(n, g[0][q], lds + dst[q]);
+  }
+  __syncthreads();
+  // lo: the five small terms in an accumulator of their own.  The MFMA aligns its
+  // products to the accumulator and cuts what falls below it, so small terms added
+  // to the large sum lean to one side (2752 k: the Gram diagonal off by -1.6e-6
+  // relative with one accumulator); beside sums of their own size they do not.
+  f32x16 lo[TW][TW];
+#pragma unroll
+  for (int i = 0; i < TW; ++i)
+#pragma unroll
+    for (int j = 0; j < TW; ++j) lo[i][j] = f32x16{};
+  // K step t: the loads of step t + 2 go out first, then behind each MFMA (32
+  // cycles) goes a part of splitting step t + 1.  Past the last step the split goes
+  // to a buffer nobody reads and the loads are left out.
+  constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
+  auto step = [&](int t, float4 (&next)[NQ], float4 (&after)[NQ]) {
+    const char* sa = lds + (t & 1) * 2 * G::OPER;
+    const char* sb = sa + G::OPER;
+    char* nx = lds + ((t + 1) & 1) * 2 * G::OPER;
+    if (t + 2 < KT) fetch(after);
+    bf16x8 av[TW][3], bv[TW][3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int i = 0; i < TW; ++i) av[i][p] = frag_k(sa, wr * WT + i * 32, p);
+#pragma unroll
+      for (int j = 0; j < TW; ++j) bv[j][p] = PX ? frag_t(sb, wc * TW + j, p) : frag_k(sb, wc * WT + j * 32, p);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < 6 * TW * TW; ++n) {
+      const int q = n / (TW * TW), i = n / TW % TW, j = n % TW;
+      f32x16& d = q == 0 ? acc[i][j] : lo[i][j];
+      d = mfma(av[i][PA[q]], bv[j][PB[q]], d);
+#pragma unroll
+      for (int u = 0; u < 2 / TW; ++u) {
+        const int x = n * (2 / TW) + u;
+        sp.part<G::PLANE>(x % 6, next[x / 6], nx + dst[x / 6]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
-    // element idx of the half, two mappings (consecutive lanes along the
-    // destination's rows): direct (r, c) = (64 h + idx / 128, idx % 128) and
-    // mirrored (r, c) = (64 h + idx % 64, idx / 64), the latter for stores
-    // along a column of the tile (a symmetric mirror, a tall block's
-    // parameter rows)
-    constexpr int PER = F_HALF * FT / F_NT;  // elements per thread and half
+  };
+  for (int t = 0; t < KT; t += 2) {
+    step(t, g[1], g[0]);
+    if (t + 1 < KT) step(t + 1, g[0], g[1]);
+  }
+  if (STAGE == NS_POLY && KT > 0) {
+    // + (b/c) A, A symmetric: the lane's four consecutive rows of one column are
+    // four consecutive columns of a row
+    const float bc = a.cb / a.cc;
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int r = r0 + wr * WT + i * 32 + 8 * q + 4 * (lane >> 5), c = c0 + wc * WT + j * 32 + (lane & 31);
+          const float4 v = *reinterpret_cast<const float4*>(A + int64_t(c) * a.mp + r);
+          lo[i][j][4 * q] = fmaf(bc, v.x, lo[i][j][4 * q]);
+          lo[i][j][4 * q + 1] = fmaf(bc, v.y, lo[i][j][4 * q + 1]);
+          lo[i][j][4 * q + 2] = fmaf(bc, v.z, lo[i][j][4 * q + 2]);
+          lo[i][j][4 * q + 3] = fmaf(bc, v.w, lo[i][j][4 * q + 3]);
+        }
+  }
+#pragma unroll
+  for (int i = 0; i < TW; ++i)
+#pragma unroll
+    for (int j = 0; j < TW; ++j) acc[i][j] += lo[i][j];
+  const float s = a.scale != nullptr ? a.scale[b] : 1.f;
+  // Output: 64 rows of the tile per pass go through LDS as T[column][row], 16-B
+  // chunks of four rows, chunk q of column c at q ^ f32_tile_swz(c).  They are read
+  // back as 4 x 4 blocks (four chunks: rows r .. r+3 of columns c .. c+3, stored as
+  // four rows of a row-major matrix, 512 B of consecutive columns per 32 lanes) or
+  // as single chunks (four rows of one column, stored along a row of the transpose);
+  // none of the accesses has a bank conflict.
+  constexpr int PASSES = FT / 64;
+  constexpr int BPT = 64 * FT / 16 / F_NT;  // 4 x 4 blocks per thread and pass
+  constexpr int CPT = 64 * FT / 4 / F_NT;   // chunks per thread and pass
+  auto chunk = [&](int c, int q) { return reinterpret_cast<float4*>(lds + c * 256 + ((q ^ f32_tile_swz(c)) << 4)); };
+  // block k of this thread: columns 4 x .. 4 x + 3, rows 4 y .. 4 y + 3 of the pass
+  auto blk = [&](int k, int& x, int& y) {
+    const int idx = threadIdx.x + F_NT * k;
+    x = idx % (FT / 4);
+    y = idx / (FT / 4);
+  };
+  // chunk k of this thread: column c, rows 4 y .. 4 y + 3 of the pass
+  auto col = [&](int k, int& c, int& y) {
+    const int idx = threadIdx.x + F_NT * k;
+    c = idx >> 4;
+    y = idx & 15;
+  };
+  auto read_blk = [&](int x, int y, float (&v)[4][4]) {  // v[row][column]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 w = *chunk(4 * x + i, y);
+      v[0][i] = w.x;
+      v[1][i] = w.y;
+      v[2][i] = w.z;
+      v[3][i] = w.w;
+    }
+  };
+  [[maybe_unused]] auto* prm =
+      STAGE == NS_PX_APPLY ? reinterpret_cast<typename TP::storage*>(a.blocks[b].param) : nullptr;
+#pragma unroll 1
+  for (int h = 0; h < PASSES; ++h) {
+    if (h) __syncthreads();  // every wave is done reading the previous pass
+    // accumulator value 4 q + e of MFMA tile (i, j) holds row WT wr + 32 i + 8 q +
+    // 4 (lane/32) + e, column WT wc + 32 j + lane%32
+    if (TW == 1 || wr == h) {
+#pragma unroll
+      for (int i = 0; i < TW; ++i)
+#pragma unroll
+        for (int j = 0; j < TW; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x16& v = acc[i][j];
+            const int r4 = (TW == 1 ? wr * 8 : 0) + i * 8 + 2 * q + (lane >> 5), c = wc * WT + j * 32 + (lane & 31);
+            *chunk(c, r4) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+          }
+    }
+    __syncthreads();
+    const int rh = r0 + 64 * h;  // first row of the pass
     if constexpr (SYM) {
-      // SYRK: A = s^2 acc; POLY: P = c (A A + (b/c) A) = b A + c A A.  A
-      // diagonal tile takes its lower triangle from the upper one: in the
-      // first half from T[c][r] (c < r < 64) and, for the 64 x 64 block
-      // below it, from the first half's mirror stores; in the second half
-      // from T[c][r] (64 <= c < r).
+      // SYRK: A = s^2 acc; POLY: P = c (A A + (b/c) A) + a I.  Each tile is stored
+      // with its mirror; a diagonal tile stores its 4 x 4 blocks above the diagonal
+      // and their mirrors, and those on it from their upper triangles.
       float* out = static_cast<float*>(a.out) + int64_t(b) * a.mp * a.mp;
       const float f = STAGE == NS_SYRK ? s * s : a.cc;
-#pragma unroll 4
-      for (int it = 0; it < PER; ++it) {
-        const int idx = threadIdx.x + F_NT * it, rl = idx >> 7, c = idx & 127, r = F_HALF * h + rl;
-        if (diag && c < F_HALF * h) continue;
-        const float v = (diag && r > c) ? T[(c - F_HALF * h) * F_ST + r] : T[rl * F_ST + c];
-        out[int64_t(r0 + r) * a.mp + c0 + c] = v * f;
-      }
-      if (!diag || h == 0) {
-#pragma unroll 4
-        for (int it = 0; it < PER; ++it) {
-          const int idx = threadIdx.x + F_NT * it, rl = idx & (F_HALF - 1), c = idx / F_HALF, r = F_HALF * h + rl;
-          if (diag && c < F_HALF) continue;
-          out[int64_t(c0 + c) * a.mp + r0 + r] = T[rl * F_ST + c] * f;  // the mirror of (r0 + r, c0 + c)
+#pragma unroll
+      for (int k = 0; k < BPT; ++k) {
+        int x, y;
+        blk(k, x, y);
+        const int r = rh + 4 * y, c = c0 + 4 * x;
+        if (diag && r > c) continue;
+        float v[4][4];
+        read_blk(x, y, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[e][i] *= f;
+        if (diag && r == c) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int i = 0; i < e; ++i) v[e][i] = v[i][e];
+            if (STAGE == NS_POLY && r + e < a.m) v[e][e] += a.ca;  // the quintic's a X: P's diagonal
+          }
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<float4*>(out + int64_t(r + e) * a.mp + c) = make_float4(v[e][0], v[e][1], v[e][2], v[e][3]);
       }
-    } else if constexpr (STAGE == NS_PX) {  // X' = s (a X + P X)
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        int c, y;
+        col(k, c, y);
+        const int r = rh + 4 * y;
+        if (diag && r >= ((c0 + c) & ~3)) continue;
+        float4 v = *chunk(c, y);
+        v.x *= f;
+        v.y *= f;
+        v.z *= f;
+        v.w *= f;
+        *reinterpret_cast<float4*>(out + int64_t(c0 + c) * a.mp + r) = v;  // the mirror
+      }
+    } else if constexpr (STAGE == NS_PX) {  // X' = s P X
       float* out = static_cast<float*>(a.out) + int64_t(b) * a.mp * a.np;
-#pragma unroll 4
-      for (int it = 0; it < PER; ++it) {
-        const int idx = threadIdx.x + F_NT * it, rl = idx >> 7, c = idx & 127;
-        out[int64_t(r0 + F_HALF * h + rl) * a.np + c0 + c] = s * T[rl * F_ST + c];
+#pragma unroll
+      for (int k = 0; k < BPT; ++k) {
+        int x, y;
+        blk(k, x, y);
+        float v[4][4];
+        read_blk(x, y, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<float4*>(out + int64_t(rh + 4 * y + e) * a.np + c0 + 4 * x) =
+              make_float4(s * v[e][0], s * v[e][1], s * v[e][2], s * v[e][3]);
       }
+    } else if (a.transposed) {
+      // PX_APPLY of a tall block: param (n x m) [column][row] += alpha X'
+      float4 v[CPT];
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        int c, y;
+        col(k, c, y);
+        v[k] = *chunk(c, y);
+      }
+      f32_update<TP, CPT>(prm, a, s, v, [&](int k, int& pr, int& pc) {
+        int c, y;
+        col(k, c, y);
+        pr = c0 + c;
+        pc = rh + 4 * y;
+      }, a.n, a.m);
     } else {
-      // PX_APPLY: param += alpha X' (un-transposed); the block is (m x n) or,
-      // tall, (n x m).  F_APPLY_BATCH elements per batch: their parameter loads
-      // are all issued before the first update is stored, so a thread waits
-      // for the load latency once per batch rather than once per element.
-      constexpr int PB = F_APPLY_BATCH;
-      static_assert(PER % PB == 0, "whole batches per thread");
-#pragma unroll 1
-      for (int it0 = 0; it0 < PER; it0 += PB) {
-        float pv[PB];
-        int64_t off[PB];
+      // ... of a wide or square block: param (m x n) [row][column]
 #pragma unroll
-        for (int q = 0; q < PB; ++q) {
-          const int idx = threadIdx.x + F_NT * (it0 + q);
-          const int rl = a.transposed ? (idx & (F_HALF - 1)) : (idx >> 7);
-          const int c = a.transposed ? (idx / F_HALF) : (idx & 127);
-          const int i = r0 + F_HALF * h + rl, j = c0 + c;
-          off[q] = i < a.m && j < a.n ? (a.transposed ? int64_t(j) * a.m + i : int64_t(i) * a.n + j) : -1;
-          pv[q] = off[q] >= 0 ? TP::load(prm, off[q]) : 0.f;
-        }
+      for (int k = 0; k < BPT; ++k) {
+        int x, y;
+        blk(k, x, y);
+        float w[4][4];
+        read_blk(x, y, w);
+        float4 v[4];
 #pragma unroll
-        for (int q = 0; q < PB; ++q) {
-          if (off[q] < 0) continue;
-          const int idx = threadIdx.x + F_NT * (it0 + q);
-          const int rl = a.transposed ? (idx & (F_HALF - 1)) : (idx >> 7);
-          const int c = a.transposed ? (idx / F_HALF) : (idx & 127);
-          TP::store(prm, off[q], fmaf(a.alpha, s * T[rl * F_ST + c], pv[q]));
-        }
+        for (int e = 0; e < 4; ++e) v[e] = make_float4(w[e][0], w[e][1], w[e][2], w[e][3]);
+        f32_update<TP, 4>(prm, a, s, v, [&](int e, int& pr, int& pc) {
+          pr = rh + 4 * y + e;
+          pc = c0 + 4 * x;
+        }, a.m, a.n);
       }
     }
   }
@@ -1139,29 +1365,40 @@ void launch_bf16(const NsArgs& a, hipStream_t s) {
   }
 }
 
-template <int STAGE, class TP>
-void launch_f32(const NsArgs& a, hipStream_t s) {
+template <int STAGE, class TP, int TW>
+void launch_f32_t(const NsArgs& a, hipStream_t s) {
+  constexpr int FT = F32Geo<TW>::FT;
+  constexpr bool SYM = STAGE == NS_SYRK || STAGE == NS_POLY;
   const int nt = a.mp / FT;
-  const int tiles = (STAGE == NS_SYRK || STAGE == NS_POLY) ? nt * (nt + 1) / 2 : nt * (a.np / FT);
-  // blocks go to grid.y (at most 65535 per launch): larger stacks in chunks
+  const int64_t tiles = SYM ? int64_t(nt) * (nt + 1) / 2 : int64_t(nt) * (a.np / FT);
   const int64_t per_x = int64_t(a.mp) * a.np, per_a = int64_t(a.mp) * a.mp;
-  const int64_t per_out = (STAGE == NS_SYRK || STAGE == NS_POLY) ? per_a : per_x;
-  for (int b0 = 0; b0 < a.N; b0 += 65535) {
+  const int64_t per_out = SYM ? per_a : per_x;
+  // at most 2^30 workgroups per launch: larger stacks in chunks of blocks
+  const int chunk = int(std::max<int64_t>(8, (int64_t(1) << 30) / tiles / 8 * 8));
+  for (int b0 = 0; b0 < a.N; b0 += chunk) {
     NsArgs c = a;
-    c.N = a.N - b0 < 65535 ? a.N - b0 : 65535;
+    c.N = std::min(a.N - b0, chunk);
     if (a.x_in) c.x_in = static_cast<const float*>(a.x_in) + b0 * per_x;
     if (a.a_in) c.a_in = static_cast<const float*>(a.a_in) + b0 * per_a;
     if (a.out) c.out = static_cast<float*>(a.out) + b0 * per_out;
     if (a.scale) c.scale = a.scale + b0;
     if (a.blocks) c.blocks = a.blocks + b0;
-    hipLaunchKernelGGL((ns_f32<STAGE, TP>), dim3(tiles, c.N), dim3(F_NT), 0, s, c);
+    hipLaunchKernelGGL((ns_f32<STAGE, TP, TW>), dim3(unsigned(8 * ((c.N + 7) / 8) * tiles)), dim3(F_NT), 0, s, c);
   }
+}
+template <int STAGE, class TP>
+void launch_f32(const NsArgs& a, hipStream_t s) {
+  constexpr bool SYM = STAGE == NS_SYRK || STAGE == NS_POLY;
+  const int nt = a.mp / 128;
+  const int64_t tiles = int64_t(a.N) * (SYM ? nt * (nt + 1) / 2 : int64_t(nt) * (a.np / 128));
+  if (tiles >= F32_FILL) launch_f32_t<STAGE, TP, 2>(a, s);
+  else launch_f32_t<STAGE, TP, 1>(a, s);
 }
 
 }  // namespace
 
-int ns_tile_m(int ns_dtype) { return ns_dtype == MMUON_BF16 ? BM : FT; }
-int ns_tile_n(int ns_dtype) { return ns_dtype == MMUON_BF16 ? 256 : FT; }  // pack tiles 256 columns
+int ns_tile_m(int ns_dtype) { return ns_dtype == MMUON_BF16 ? BM : F_PAD; }
+int ns_tile_n(int ns_dtype) { return ns_dtype == MMUON_BF16 ? 256 : F_PAD; }  // pack tiles 256 columns
 int ns_tile_k(int ns_dtype) { return ns_dtype == MMUON_BF16 ? BK : FK; }
 
 int launch_ns_stage(const NsArgs& a, int stage, int ns_dtype, int param_dtype, hipStream_t s) {

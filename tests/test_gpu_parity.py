@@ -141,6 +141,28 @@ def test_ns_fp32_against_fp64_truth(shape):
     assert e.max() < 1e-5, (e, e_ref)
 
 
+# both tile sizes of the fp32 kernels (128-wide from 256 such tiles per launch), K extents that end in an odd or a
+# single step, and 64-wide tiles that hold only padding
+@pytest.mark.parametrize("shape", [(26, 512, 512), (256, 104, 128), (60, 200, 264), (64, 264, 136), (3, 150, 200),
+                                   (2, 8, 16), (1, 16, 8), (2, 130, 130)], ids=lambda s: "x".join(map(str, s)))
+def test_ns_fp32_tiles_against_fp64_truth(shape):
+    """The bar of the fp32 path, 1e-5; one block of the stack set to NaN and one holding an infinity come out
+    non-finite and leave the others untouched."""
+    gen = torch.Generator().manual_seed(21)
+    g = (torch.randn(shape, generator=gen) * 1e-3).to(DEV)
+    ours = run_ns_only(g, None)
+    e = rel_fro(ours, ns_fp64(g.cpu().double()))
+    print(f"NS fp32 {shape}: vs fp64 {e.max():.2e}")
+    assert e.max() < 1e-5, e
+    if shape[0] > 2:
+        bad = g.clone()
+        bad[0] = float("nan")
+        bad[2, 1, 3] = float("inf")
+        out = run_ns_only(bad, None)
+        assert not torch.isfinite(out[0]).any() and not torch.isfinite(out[2]).any()
+        assert torch.equal(out[1], ours[1]) and torch.equal(out[3:], ours[3:])
+
+
 @pytest.mark.parametrize("shape", [(2, 256, 256), (2, 256, 688), (2, 688, 256)], ids=lambda s: "x".join(map(str, s)))
 def test_ns_zero_block_gives_zero(shape):
     """A zero block stays zero, alone and beside a non-zero block of the same
