@@ -394,7 +394,7 @@ __device__ __forceinline__ void gemm_work(const GemmArgs& a, uint16_t* lds, int 
     char* stage = reinterpret_cast<char*>(lds);
     barrier();  // every wave is done with the ring
     stage_acc(stage, acc);
-    barrier();
+    barrier_after_lds_writes();
     const GOut& c = a.c;
     char* cb = c.base + int64_t(g) * c.bstride;
     const int wshift = 8 - c.log2l;

@@ -109,6 +109,13 @@ __device__ __forceinline__ void barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Workgroup barrier after LDS writes that other waves read: s_barrier alone does not
+// wait for this wave's own LDS operations, and the compiler adds no wait on gfx950.
+__device__ __forceinline__ void barrier_after_lds_writes() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  barrier();
+}
+
 // ----- LDS layouts --------------------------------------------------------
 // K-form slice [rows][32 k] (consecutive rows of one panel): a row is four
 // 16-B chunks; chunk c of row r sits in slot c ^ ((r >> 2) & 3), so the 16 rows

@@ -631,7 +631,7 @@ __device__ __forceinline__ void sym_work(const NsArgs& a, uint16_t* lds, int v) 
   barrier();  // every wave is done with the ring
   // POLY: a on the diagonal of the m valid rows (the padding stays zero)
   stage_tile(stage, acc, f, diag, STAGE == NS_POLY ? a.ca : 0.f, STAGE == NS_POLY ? a.m - r0 : 0);
-  barrier();
+  barrier_after_lds_writes();
   if (!diag) {
     // upper tile C[r0 + i][c0 + r] = T[r][i]
     uint16_t* dst = out + (c0 / PANEL) * pstride + int64_t(r0) * PANEL;
@@ -767,7 +767,7 @@ __device__ __forceinline__ void px_work(const NsArgs& a, uint16_t* lds, int v) {
   }
   barrier();  // every wave is done with the ring
   stage_tile(stage, acc, s);
-  barrier();
+  barrier_after_lds_writes();
   if (STAGE == NS_PX) {
     // X'[r0 + i][c0 + r] = T[r][i]
     uint16_t* dst = static_cast<uint16_t*>(a.out) + int64_t(b) * a.mp * a.np + (c0 / PANEL) * pstride +
