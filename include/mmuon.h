@@ -382,11 +382,19 @@ int mmuon_butterfly_fwd(const mmuon_butterfly_args* a, void* stream);
 int mmuon_butterfly_bwd(const mmuon_butterfly_args* a, void* stream);
 /* Workspace bytes the backward needs for these shapes (x, pointers unused). */
 size_t mmuon_butterfly_workspace(const mmuon_butterfly_args* a);
+/* The same products with out and dout in the layer's feature order, (tokens,
+   s * nblocks) with feature j * nblocks + ll = column j of block ll: the
+   layer's own output and gradient (monarch_ops.py:105-114 transposes them in
+   passes of its own). */
+int mmuon_butterfly_linear_fwd(const mmuon_butterfly_args* a, void* stream);
+int mmuon_butterfly_linear_bwd(const mmuon_butterfly_args* a, void* stream);
+size_t mmuon_butterfly_linear_workspace(const mmuon_butterfly_args* a);
 
 /* Thread-local message of the last failing call ("" if none). */
 const char* mmuon_last_error(void);
 
-/* ABI version: bumped on any change to this header. */
+/* ABI version: bumped when a declaration of this header changes (not when one
+   is added). */
 int mmuon_abi_version(void);
 
 #ifdef __cplusplus

@@ -130,6 +130,9 @@ SIGNATURES = {
     "mmuon_butterfly_fwd": (C.c_int, [C.POINTER(ButterflyArgs), C.c_void_p]),
     "mmuon_butterfly_bwd": (C.c_int, [C.POINTER(ButterflyArgs), C.c_void_p]),
     "mmuon_butterfly_workspace": (C.c_size_t, [C.POINTER(ButterflyArgs)]),
+    "mmuon_butterfly_linear_fwd": (C.c_int, [C.POINTER(ButterflyArgs), C.c_void_p]),
+    "mmuon_butterfly_linear_bwd": (C.c_int, [C.POINTER(ButterflyArgs), C.c_void_p]),
+    "mmuon_butterfly_linear_workspace": (C.c_size_t, [C.POINTER(ButterflyArgs)]),
 }
 
 _lib = None

@@ -534,7 +534,7 @@ namespace {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-int check_butterfly(const mmuon_butterfly_args* a, bool bwd) {
+int check_butterfly(const mmuon_butterfly_args* a, bool bwd, bool features = false) {
   if (a == nullptr) return fail(MMUON_EINVAL, "null butterfly arguments");
   if (a->dtype != MMUON_BF16) return fail(MMUON_EINVAL, "butterfly: dtype must be MMUON_BF16 (got %d)", a->dtype);
   const int nb = a->nblocks;
@@ -568,9 +568,9 @@ int check_butterfly(const mmuon_butterfly_args* a, bool bwd) {
     return fail(MMUON_EINVAL, "butterfly: null or unaligned backward pointer");
   if ((reinterpret_cast<uintptr_t>(a->workspace) & 255) != 0)
     return fail(MMUON_EINVAL, "butterfly: workspace must be 256-B aligned");
-  if (a->workspace_bytes < mmuon::butterfly_workspace(*a))
-    return fail(MMUON_EINVAL, "butterfly: workspace of %zu bytes, %zu needed", a->workspace_bytes,
-                mmuon::butterfly_workspace(*a));
+  const size_t need = features ? mmuon::butterfly_linear_workspace(*a) : mmuon::butterfly_workspace(*a);
+  if (a->workspace_bytes < need)
+    return fail(MMUON_EINVAL, "butterfly: workspace of %zu bytes, %zu needed", a->workspace_bytes, need);
   return MMUON_OK;
 }
 
@@ -583,15 +583,32 @@ size_t mmuon_butterfly_workspace(const mmuon_butterfly_args* a) {
   return mmuon::butterfly_workspace(*a);
 }
 
+size_t mmuon_butterfly_linear_workspace(const mmuon_butterfly_args* a) {
+  if (a == nullptr || a->nblocks <= 0 || a->q <= 0 || a->p <= 0 || a->s <= 0 || a->tokens < 0) return 0;
+  return mmuon::butterfly_linear_workspace(*a);
+}
+
+int mmuon_butterfly_linear_fwd(const mmuon_butterfly_args* a, void* stream) {
+  if (int rc = check_butterfly(a, false)) return rc;
+  mmuon::launch_butterfly_fwd(*a, true, static_cast<hipStream_t>(stream));
+  return check_launch("butterfly forward");
+}
+
+int mmuon_butterfly_linear_bwd(const mmuon_butterfly_args* a, void* stream) {
+  if (int rc = check_butterfly(a, true, true)) return rc;
+  mmuon::launch_butterfly_bwd(*a, true, static_cast<hipStream_t>(stream));
+  return check_launch("butterfly backward");
+}
+
 int mmuon_butterfly_fwd(const mmuon_butterfly_args* a, void* stream) {
   if (int rc = check_butterfly(a, false)) return rc;
-  mmuon::launch_butterfly_fwd(*a, static_cast<hipStream_t>(stream));
+  mmuon::launch_butterfly_fwd(*a, false, static_cast<hipStream_t>(stream));
   return check_launch("butterfly forward");
 }
 
 int mmuon_butterfly_bwd(const mmuon_butterfly_args* a, void* stream) {
   if (int rc = check_butterfly(a, true)) return rc;
-  mmuon::launch_butterfly_bwd(*a, static_cast<hipStream_t>(stream));
+  mmuon::launch_butterfly_bwd(*a, false, static_cast<hipStream_t>(stream));
   return check_launch("butterfly backward");
 }
 

@@ -19,15 +19,25 @@
 // back in place.  bf16 operands, fp32 accumulation, bf16 results (the rounding
 // points of the reference's bf16 bmms: out1, out, dt, dx, dw1, dw2).
 //
-// One GEMM kernel serves all six products: 256 x 256 output tiles per
-// 512-thread workgroup, the MFMA pipeline and LDS slice forms of mfma_tile.hpp,
+// One GEMM kernel serves all six products, in 256-, 128- and 64-wide tiles (gemm_plan
+// picks by the shapes): the MFMA pipeline and LDS slice forms of mfma_tile.hpp,
 // operands K-major (K form) or MN-major (T form, read transposed with
 // ds_read_b64_tr_b16), staged by buffer loads straight into LDS.  A buffer load
 // whose lane offset is beyond the resource's range returns zeros, which pads
-// partial tiles (token counts and block sides that are not multiples of 256)
+// partial tiles (token counts and block sides that are not multiples of the tile)
 // without branches in the loop.  The weight-gradient products contract over the
 // tokens and have few output tiles; they split K and reduce the fp32 partials
-// in a fixed order (deterministic).
+// in a fixed order (deterministic).  The layer's own output is in feature order,
+// (B, s l) with feature j l + ll = out[b][ll][j]: F2 can store it so directly, and the
+// backward splits dout's blocks in one pass (to_blocks_kernel).
+//
+// What bounds it, one 6.89B up-projection (4 x 1024 x 1024, 4 x 2752 x 1024) at 4096
+// tokens, forward + backward 563 -> 465 us with the output stored in feature order
+// (two strided copies of 63-72 us before, one pass of 27-35 now): the 256-wide products
+// spend 8 us of a 45 us round filling and draining the pipeline, and read and write LDS
+// as long as their MFMAs run.  At 4096 tokens of 4 x 512 x 512 the 128-wide tiles took
+// the six products from 157 to 121 us, at 1000 tokens of 2 x 256 x 256 the 64-wide ones
+// from 125 to 52, at 8 tokens of the 6.89B layer (two products) from 53 to 22.
 #include <algorithm>
 #include <atomic>
 
@@ -123,194 +133,234 @@ struct GOut {
   int32_t log2l;
 };
 
+// What the epilogue writes: bf16 rows (c), fp32 partials, or bf16 in feature order
+// (column j of batch g at base + row rstride + (j G + g) 2).
+enum { OUT_TILE = 0, OUT_PARTIAL = 1, OUT_FEATURES = 2 };
 struct GemmArgs {
   GOp a, b;        // row operand (M x K), column operand (N x K)
   GOut c;          // bf16 result (partial == null)
   float* partial;  // split-K: fp32 partials [S][G][M][N]
   int M, N, K, G, S;
   int kchunk;      // K per split, a multiple of BK
+  int tile;        // tile geometry
   int tiles_m, tiles_n;
   int vtiles;      // virtual tiles: 8 XCDs x ceil(G * S * tiles_m / 8) groups x tiles_n
 };
 
 // ---------------------------------------------------------------------------
+// Tile geometries: GM x GN waves, each WI x WJ MFMA tiles of 32 x 32; RING slices
+// of 32 k in LDS.
+// ---------------------------------------------------------------------------
+template <int GM_, int GN_, int WI_, int WJ_, int RING_>
+struct Geo {
+  static constexpr int GM = GM_, GN = GN_, WI = WI_, WJ = WJ_, RING = RING_;
+  static constexpr int NW = GM * GN, NTH = 64 * NW;
+  static constexpr int BM = 32 * WI * GM, BN = 32 * WJ * GN;
+  static constexpr int RSLB = BM * BK * 2, SLOTB = (BM + BN) * BK * 2;  // bytes of a row slice, of a slot
+  static constexpr int RL = BM / 16 / NW, CL = BN / 16 / NW;            // 1 KiB loads per wave and operand slice
+  static constexpr int DMA = RL + CL;
+  static constexpr int LDS = RING * SLOTB;
+  static constexpr int PER_CU = 160 * 1024 / LDS < 4 ? 160 * 1024 / LDS : 4;  // workgroups resident per CU
+  static_assert(RL * NW * 16 == BM && CL * NW * 16 == BN, "whole loads per wave");
+  static_assert(BM * BN * 2 <= LDS && LDS <= 160 * 1024, "the staged tile fits in the ring");
+  // Staged tile T[j][i] = D[i][j]: rows of BM bf16, 16-B chunk c of row r at c ^ g(r),
+  // g distinct over the rows that one access touches (mfma_tile.hpp, tile_off; rows of
+  // 128 B take two per pass over the banks)
+  static __device__ __forceinline__ uint32_t tile_at(int r, int c) {
+    const int g = BM >= 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (r >> 1) & 7;
+    return uint32_t(r * BM * 2 + (((c >> 3) ^ g) << 4) + ((c & 7) << 1));
+  }
+};
+
+// ---------------------------------------------------------------------------
 // The pipelined main loop (the NS kernels' schedule with both operand forms
 // fixed per launch): slice kt in ring slot kt % RING, RING - 2 slices in flight
-// behind the one being read, fragment reads and buffer loads interleaved one
-// per MFMA.  (A fifth slot, the whole LDS, measured slightly slower.)
+// behind the one being read, fragment reads and buffer loads interleaved with the
+// MFMAs.  (256 x 256 tiles: a fifth slot, the whole LDS, measured slightly slower.)
 // ---------------------------------------------------------------------------
-constexpr int RING = 4;
-constexpr int RING_ELEMS = RING * SLOT;
-static_assert(RING_ELEMS * 2 <= 160 * 1024 && RING_ELEMS >= BN * 256, "ring and staged tile fit the LDS");
-template <bool AT, bool BT>
+template <class GE, bool AT, bool BT>
 struct GPipe {
-  static_assert(RDMA == 2 && CDMA == 2, "two buffer loads per thread and operand slice");
+  static constexpr int RING = GE::RING, WI = GE::WI, WJ = GE::WJ, NM = WI * WJ, NR = WI + WJ;
+  struct Fr {
+    bf16x8 r[WI];
+    bf16x8 c[WJ];
+  };
+  typedef f32x16 Acc[WI][WJ];
   const char* abase;  // row operand at (tile row 0, k = 0) of this batch
   const char* bbase;
   GOpK ak, bk;        // K addressing of the two operands
-  uint32_t loff[4];   // per-lane byte offsets of the four loads (OOB: beyond the extent)
+  uint32_t loff[GE::DMA];  // per-lane byte offsets of the loads (OOB: beyond the extent)
   int kbeg, kend, KT;
   int wave, lane, wm, wn;
-  uint16_t* lds;
+  char* lds;
   uint32_t lds0;
   uint32_t kfrag[BK / 16];
   uint32_t tfrag_r, tfrag_c;
 
-  __device__ __forceinline__ const uint16_t* slot(int kt) const { return lds + (kt % RING) * SLOT; }
-
-  // K delta of this lane's load q within a slice: K form, its 8-element chunk;
-  // T form, its k row
-  template <bool T>
-  __device__ __forceinline__ int kdelta(int q) const {
-    return T ? 16 * q + (lane >> 2) : 8 * ((lane & 3) ^ ((lane >> 4) & 3));
+  __device__ __forceinline__ const uint16_t* slot(int kt) const {
+    return reinterpret_cast<const uint16_t*>(lds + (uint32_t(kt) % RING) * GE::SLOTB);
   }
 
-  // Load Q (0, 1: row operand; 2, 3: column operand) of slice src_kt into the
-  // slot of slice slot_kt.  K form: operand rows 16 (2w + q) + lane/4, chunk
-  // (lane%4) ^ ((lane>>4)&3); T form: k rows 16 q + lane/4 of the slice,
-  // MN 32 w + 8 (lane%4).  Either way the load lands at byte (2w + q) * 1024 of
-  // the operand's slice.
+  // Load Q (row operand first) of slice src_kt into the slot of slice slot_kt.
+  // Load u = RL wave + Q (CL wave + Q - RL) of the operand's BM / 16 (BN / 16).
+  // K form: operand rows 16 u + lane/4, chunk (lane%4) ^ ((lane>>4)&3); T form: k rows
+  // 16 (u%2) + lane/4 of the slice, MN 32 (u/2) + 8 (lane%4).  Either way the load
+  // lands at byte 1024 u of the operand's slice.
   template <int Q>
   __device__ __forceinline__ void issue_one(int src_kt, int slot_kt) const {
-    constexpr int q = Q & 1;
-    constexpr bool T = Q < 2 ? AT : BT;
-    const uint32_t dst = lds0 + (slot_kt % RING) * SLOT * 2 + (Q < 2 ? 0 : RSLICE * 2) + (2 * wave + q) * 1024;
+    constexpr bool ROW = Q < GE::RL;
+    constexpr bool T = ROW ? AT : BT;
+    const int u = ROW ? GE::RL * wave + Q : GE::CL * wave + Q - GE::RL;
+    const uint32_t dst = lds0 + (uint32_t(slot_kt) % RING) * GE::SLOTB + (ROW ? 0 : GE::RSLB) + u * 1024;
     const int k0 = kbeg + src_kt * BK;
-    const char* sb = (Q < 2 ? abase : bbase) + k_off(Q < 2 ? ak : bk, k0);
+    const char* sb = (ROW ? abase : bbase) + k_off(ROW ? ak : bk, k0);
     uint32_t voff = loff[Q];
     const int rem = kend - k0;
-    if (rem < BK && kdelta<T>(q) >= rem) voff = OOB;
+    if (rem < BK) {
+      // K delta of this lane's load within the slice: K form, its 8-element chunk; T form, its k row
+      const int kd = T ? 16 * (u & 1) + (lane >> 2) : 8 * ((lane & 3) ^ ((lane >> 4) & 3));
+      if (kd >= rem) voff = OOB;
+    }
     bdma16(buffer_rsrc(sb), voff, dst);
   }
+  template <int Q0, int Q1>
   __device__ __forceinline__ void issue(int src_kt, int slot_kt) const {
-    issue_one<0>(src_kt, slot_kt);
-    issue_one<1>(src_kt, slot_kt);
-    issue_one<2>(src_kt, slot_kt);
-    issue_one<3>(src_kt, slot_kt);
+    if constexpr (Q0 < Q1) {
+      issue_one<Q0>(src_kt, slot_kt);
+      issue<Q0 + 1, Q1>(src_kt, slot_kt);
+    }
   }
 
   template <int KK, int G>
-  __device__ __forceinline__ void load_one(int kt, Frags& f) const {
+  __device__ __forceinline__ void load_one(int kt, Fr& f) const {
     const uint16_t* sr = slot(kt);
-    const uint16_t* sc = sr + RSLICE;
-    if constexpr (G < TMJ)
-      f.c[G] = BT ? frag_rowmajor_tr(sc, tfrag_c + G * 2048, KK) : frag_kmajor(sc, kfrag[KK], wn * WN + G * 32);
+    const uint16_t* sc = sr + GE::RSLB / 2;
+    if constexpr (G < WJ)
+      f.c[G] = BT ? frag_rowmajor_tr(sc, tfrag_c + G * 2048, KK) : frag_kmajor(sc, kfrag[KK], (wn * WJ + G) * 32);
     else
-      f.r[G - TMJ] = AT ? frag_rowmajor_tr(sr, tfrag_r + (G - TMJ) * 2048, KK)
-                        : frag_kmajor(sr, kfrag[KK], wm * WM + (G - TMJ) * 32);
+      f.r[G - WJ] = AT ? frag_rowmajor_tr(sr, tfrag_r + (G - WJ) * 2048, KK)
+                       : frag_kmajor(sr, kfrag[KK], (wm * WI + G - WJ) * 32);
+  }
+  template <int KK, int G0, int G1>
+  __device__ __forceinline__ void load(int kt, Fr& f) const {
+    if constexpr (G0 < G1) {
+      load_one<KK, G0>(kt, f);
+      load<KK, G0 + 1, G1>(kt, f);
+    }
   }
 
-  __device__ __forceinline__ void body(int kt, Frags& fa, Frags& fb, f32x16 (&acc)[TMI][TMJ]) const {
-    static_assert(TMI * TMJ == 8 && SLICE_DMA <= 8 && TMI + TMJ <= 8, "one read / load per MFMA");
-#define MMUON_GSTEP0(g)                                                                      \
-    acc[(g) / TMJ][(g) % TMJ] = mfma(fa.r[(g) / TMJ], fa.c[(g) % TMJ], acc[(g) / TMJ][(g) % TMJ]); \
-    if constexpr ((g) < TMI + TMJ) load_one<1, (g)>(kt, fb);                                 \
-    __builtin_amdgcn_sched_barrier(0);
-    MMUON_GSTEP0(0) MMUON_GSTEP0(1) MMUON_GSTEP0(2) MMUON_GSTEP0(3)
-    MMUON_GSTEP0(4) MMUON_GSTEP0(5) MMUON_GSTEP0(6) MMUON_GSTEP0(7)
-#undef MMUON_GSTEP0
-    wait_vm<(RING - 3) * SLICE_DMA>();  // slice kt+1 landed
+  // MFMA g of a k step, with its share of the fragment reads of the next step and,
+  // in the second k step, of the direct loads
+  template <int KK, int g>
+  __device__ __forceinline__ void half(int kt, int src, int slt, const Fr& f, Fr& n, Acc& acc) const {
+    if constexpr (g < NM) {
+      acc[g / WJ][g % WJ] = mfma(f.r[g / WJ], f.c[g % WJ], acc[g / WJ][g % WJ]);
+      if constexpr (KK == 0) {
+        load<1, g * NR / NM, (g + 1) * NR / NM>(kt, n);
+      } else {
+        load<0, g * NR / NM, (g + 1) * NR / NM>(kt + 1, n);
+        issue<g * GE::DMA / NM, (g + 1) * GE::DMA / NM>(src, slt);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      half<KK, g + 1>(kt, src, slt, f, n, acc);
+    }
+  }
+
+  __device__ __forceinline__ void body(int kt, Fr& fa, Fr& fb, Acc& acc) const {
+    half<0, 0>(kt, 0, 0, fa, fb, acc);
+    wait_vm<(RING - 3) * GE::DMA>();  // slice kt+1 landed
     barrier();
     const int src = kt + RING - 1 < KT ? kt + RING - 1 : KT - 1;
-    const int slt = kt + RING - 1;
-#define MMUON_GSTEP1(g)                                                                      \
-    acc[(g) / TMJ][(g) % TMJ] = mfma(fb.r[(g) / TMJ], fb.c[(g) % TMJ], acc[(g) / TMJ][(g) % TMJ]); \
-    if constexpr ((g) < TMI + TMJ) load_one<0, (g)>(kt + 1, fa);                             \
-    if constexpr ((g) < SLICE_DMA) issue_one<(g)>(src, slt);                                 \
-    __builtin_amdgcn_sched_barrier(0);
     // raised wave priority from the barrier to the end of k step 1, so the
     // SIMD's wave still in this phase wins issue over one already in the next
     // step and catches up before the next barrier
     __builtin_amdgcn_s_setprio(1);
-    MMUON_GSTEP1(0) MMUON_GSTEP1(1) MMUON_GSTEP1(2) MMUON_GSTEP1(3)
-    MMUON_GSTEP1(4) MMUON_GSTEP1(5) MMUON_GSTEP1(6) MMUON_GSTEP1(7)
-#undef MMUON_GSTEP1
+    half<1, 0>(kt, src, kt + RING - 1, fb, fa, acc);
     __builtin_amdgcn_s_setprio(0);
   }
 
-  __device__ __forceinline__ void run(f32x16 (&acc)[TMI][TMJ]) const {
+  __device__ __forceinline__ void run(Acc& acc) const {
 #pragma unroll
-    for (int i = 0; i < TMI; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
-      for (int j = 0; j < TMJ; ++j) acc[i][j] = f32x16{};
+      for (int j = 0; j < WJ; ++j) acc[i][j] = f32x16{};
 #pragma unroll
-    for (int q = 0; q < RING - 1; ++q) issue(q < KT ? q : KT - 1, q);
-    wait_vm<(RING - 2) * SLICE_DMA>();  // slice 0 landed
+    for (int q = 0; q < RING - 1; ++q) issue<0, GE::DMA>(q < KT ? q : KT - 1, q);
+    wait_vm<(RING - 2) * GE::DMA>();  // slice 0 landed
     barrier();
-    Frags fa, fb;
-    load_one<0, 0>(0, fa);
-    load_one<0, 1>(0, fa);
-    load_one<0, 2>(0, fa);
-    load_one<0, 3>(0, fa);
-    load_one<0, 4>(0, fa);
-    load_one<0, 5>(0, fa);
+    Fr fa, fb;
+    load<0, 0, NR>(0, fa);
     for (int kt = 0; kt < KT; ++kt) body(kt, fa, fb, acc);
     wait_vm<0>();  // the refills of the last steps land before the ring is reused
   }
 };
 
-// Per-lane byte offset of load q of an operand (tile origin mn0), OOB beyond
+// Per-lane byte offset of load u of an operand (tile origin mn0), OOB beyond
 // its extent.
 template <bool T>
-__device__ __forceinline__ uint32_t lane_offset(const GOp& o, int mn0, int wave, int lane, int q) {
+__device__ __forceinline__ uint32_t lane_offset(const GOp& o, int mn0, int u, int lane) {
   int mn;
   int64_t off;
   if (T) {
-    mn = mn0 + 32 * wave + 8 * (lane & 3);
-    off = int64_t(16 * q + (lane >> 2)) * o.kstride;
+    mn = mn0 + 32 * (u >> 1) + 8 * (lane & 3);
+    off = int64_t(16 * (u & 1) + (lane >> 2)) * o.kstride;
   } else {
-    mn = mn0 + 16 * (2 * wave + q) + (lane >> 2);
+    mn = mn0 + 16 * u + (lane >> 2);
     off = int64_t((lane & 3) ^ ((lane >> 4) & 3)) * 16;
   }
   if (mn >= o.extent) return OOB;
   return uint32_t(off + mn_off(o, mn) - mn_off(o, mn0));
 }
 
-// Accumulators -> the staging area as T[j][i] = D[i][j] (tile_off layout), bf16.
-__device__ __forceinline__ void stage_acc(char* stage, const f32x16 (&acc)[TMI][TMJ]) {
+// Accumulators -> the staging area as T[j][i] = D[i][j], bf16.
+template <class GE>
+__device__ __forceinline__ void stage_acc(char* stage, const f32x16 (&acc)[GE::WI][GE::WJ]) {
   const int tid = fresh_tid();
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / NWN, wn = wave % NWN;
+  const int wm = wave / GE::GN, wn = wave % GE::GN;
 #pragma unroll
-  for (int i = 0; i < TMI; ++i)
+  for (int i = 0; i < GE::WI; ++i)
 #pragma unroll
-    for (int j = 0; j < TMJ; ++j)
+    for (int j = 0; j < GE::WJ; ++j)
 #pragma unroll
       for (int qg = 0; qg < 4; ++qg) {
         const f32x16& v = acc[i][j];
-        const int row = wn * WN + j * 32 + (lane & 31);
-        const int col = wm * WM + i * 32 + qg * 8 + (lane >> 5) * 4;
-        *reinterpret_cast<uint2*>(stage + tile_off(row, col)) =
+        const int row = (wn * GE::WJ + j) * 32 + (lane & 31);
+        const int col = (wm * GE::WI + i) * 32 + qg * 8 + (lane >> 5) * 4;
+        *reinterpret_cast<uint2*>(stage + GE::tile_at(row, col)) =
             make_uint2(f2bf2(v[qg * 4], v[qg * 4 + 1]), f2bf2(v[qg * 4 + 2], v[qg * 4 + 3]));
       }
 }
 
 // Staged tile -> destination rows.  Tile column order is permuted by the
-// riffle: destination position dc (plane dc / (256/l), column dc % (256/l))
-// holds tile column (dc % (256/l)) l + dc / (256/l).  ds_read_b64_tr_b16 on
+// riffle: destination position dc (plane dc / (BN/l), column dc % (BN/l))
+// holds tile column (dc % (BN/l)) l + dc / (BN/l).  ds_read_b64_tr_b16 on
 // 16-lane groups: lanes 4e..4e+3 address staged row (tile column) R(e), four
 // consecutive tile rows each, and lane i receives D[i0 + i][R(0..3)].  A wave
 // task covers 16 tile rows x 64 destination columns; a lane writes two 16-B
-// chunks.  fn(row, dc, uint4) stores destination columns dc .. dc+7 of a row.
-template <class Fn>
+// chunks.  fn(row, dc, uint4) stores destination columns dc .. dc+7 of a row
+// (BN / l is a multiple of 8, so they lie in one plane).
+constexpr int log2i(int n) { return n <= 1 ? 0 : 1 + log2i(n / 2); }
+template <class GE, class Fn>
 __device__ __forceinline__ void write_tile(const char* stage, int log2l, Fn&& fn) {
   const int tid = fresh_tid();
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, grp = lane >> 4;
-  const int wshift = 8 - log2l, wmask = (1 << wshift) - 1;  // plane width 256 / l
+  const int wshift = log2i(GE::BN) - log2l, wmask = (1 << wshift) - 1;  // plane width BN / l
   auto trow = [&](int dc) { return ((dc & wmask) << log2l) | (dc >> wshift); };
+  constexpr int RB = GE::BM / 16;  // row blocks
 #pragma unroll 2
-  for (int it = 0; it < 16 * 4 / NWAVES; ++it) {
-    const int task = wave + NWAVES * it;
-    const int i0 = (task & 15) * 16;
+  for (int it = 0; it < RB * (GE::BN / 64) / GE::NW; ++it) {
+    const int task = wave + GE::NW * it;
+    const int i0 = (task % RB) * 16;
     const int tc = i0 + ((l16 & 3) << 2);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int dc = (task >> 4) * 64 + grp * 16 + h * 8;
+      const int dc = (task / RB) * 64 + grp * 16 + h * 8;
       const i16x4 lo =
-          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(stage + tile_off(trow(dc + (l16 >> 2)), tc)));
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(stage + GE::tile_at(trow(dc + (l16 >> 2)), tc)));
       const i16x4 hi =
-          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(stage + tile_off(trow(dc + 4 + (l16 >> 2)), tc)));
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(stage + GE::tile_at(trow(dc + 4 + (l16 >> 2)), tc)));
       uint4 v;
       v.x = uint32_t(uint16_t(lo[0])) | (uint32_t(uint16_t(lo[1])) << 16);
       v.y = uint32_t(uint16_t(lo[2])) | (uint32_t(uint16_t(lo[3])) << 16);
@@ -327,30 +377,42 @@ __device__ __forceinline__ void write_tile(const char* stage, int log2l, Fn&& fn
 // runs on XCD v % 8), so the tiles of one XCD share one batch's column operand
 // and few row bands, and each operand block is fetched from HBM by one or two
 // XCDs rather than by all eight.
+// Feature-order output: a group is the G tiles (one per batch) of one (tm, tn), which
+// write the same lines; groups are numbered tn fastest.
+template <bool FEATURES>
 __device__ __forceinline__ bool decode_gemm_tile(const GemmArgs& a, int v, int& g, int& sp, int& tm, int& tn) {
   const int xcd = v & 7, local = v >> 3;
-  const int ngroups = a.G * a.S * a.tiles_m;
+  const int per = FEATURES ? a.G : a.tiles_n;  // tiles of a group
+  const int ngroups = FEATURES ? a.tiles_m * a.tiles_n : a.G * a.S * a.tiles_m;
   const int gpx = (ngroups + 7) / 8;  // groups per XCD
-  const int lg = local / a.tiles_n;
+  const int lg = local / per;
   const int grp = xcd * gpx + lg;
-  tn = local % a.tiles_n;
+  const int in = local % per;
   if (lg >= gpx || grp >= ngroups) return false;
-  tm = grp % a.tiles_m;
-  sp = (grp / a.tiles_m) % a.S;
-  g = grp / (a.tiles_m * a.S);
+  if constexpr (FEATURES) {
+    g = in;
+    sp = 0;
+    tn = grp % a.tiles_n;
+    tm = grp / a.tiles_n;
+  } else {
+    tn = in;
+    tm = grp % a.tiles_m;
+    sp = (grp / a.tiles_m) % a.S;
+    g = grp / (a.tiles_m * a.S);
+  }
   return true;
 }
 
-template <bool AT, bool BT, bool SPLIT>
-__device__ __forceinline__ void gemm_work(const GemmArgs& a, uint16_t* lds, int v) {
+template <class GE, bool AT, bool BT, int OUT>
+__device__ __forceinline__ void gemm_work(const GemmArgs& a, char* lds, int v) {
   int g, sp, tm, tn;
-  if (!decode_gemm_tile(a, v, g, sp, tm, tn)) return;
-  const int m0 = tm * BM, n0 = tn * BN;
-  GPipe<AT, BT> p;
+  if (!decode_gemm_tile<OUT == OUT_FEATURES>(a, v, g, sp, tm, tn)) return;
+  const int m0 = tm * GE::BM, n0 = tn * GE::BN;
+  GPipe<GE, AT, BT> p;
   p.lane = threadIdx.x & 63;
   p.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  p.wm = p.wave / NWN;
-  p.wn = p.wave % NWN;
+  p.wm = p.wave / GE::GN;
+  p.wn = p.wave % GE::GN;
   p.ak = k_addr(a.a);
   p.bk = k_addr(a.b);
   p.abase = a.a.base + int64_t(g) * a.a.bstride + mn_off(a.a, m0);
@@ -358,48 +420,69 @@ __device__ __forceinline__ void gemm_work(const GemmArgs& a, uint16_t* lds, int 
   p.kbeg = sp * a.kchunk;
   p.kend = min(a.K, p.kbeg + a.kchunk);
   p.KT = (p.kend - p.kbeg + BK - 1) / BK;
-  p.loff[0] = lane_offset<AT>(a.a, m0, p.wave, p.lane, 0);
-  p.loff[1] = lane_offset<AT>(a.a, m0, p.wave, p.lane, 1);
-  p.loff[2] = lane_offset<BT>(a.b, n0, p.wave, p.lane, 0);
-  p.loff[3] = lane_offset<BT>(a.b, n0, p.wave, p.lane, 1);
+#pragma unroll
+  for (int q = 0; q < GE::RL; ++q) p.loff[q] = lane_offset<AT>(a.a, m0, GE::RL * p.wave + q, p.lane);
+#pragma unroll
+  for (int q = 0; q < GE::CL; ++q) p.loff[GE::RL + q] = lane_offset<BT>(a.b, n0, GE::CL * p.wave + q, p.lane);
   p.lds = lds;
   p.lds0 = lds_addr(lds);
 #pragma unroll
   for (int kk = 0; kk < BK / 16; ++kk) p.kfrag[kk] = kmajor_frag_base(kk, p.lane);
-  p.tfrag_r = rowmajor_frag_base(p.wm * TMI, p.lane);
-  p.tfrag_c = rowmajor_frag_base(p.wn * TMJ, p.lane);
-  f32x16 acc[TMI][TMJ];
+  p.tfrag_r = rowmajor_frag_base(p.wm * GE::WI, p.lane);
+  p.tfrag_c = rowmajor_frag_base(p.wn * GE::WJ, p.lane);
+  f32x16 acc[GE::WI][GE::WJ];
   p.run(acc);
 
-  if constexpr (SPLIT) {
+  if constexpr (OUT == OUT_FEATURES) {
+    // bf16 straight from the accumulators: column j of batch g is feature j G + g of
+    // the row, so a wave store puts 2 B at 32 places 2 G B apart in two rows; the
+    // other batches' tiles fill the rest of the lines in the same L2 (measured: as
+    // fast as the staged stores, and no interleaving pass follows)
+    const GOut& c = a.c;
+    const int lane = p.lane;
+#pragma unroll
+    for (int j = 0; j < GE::WJ; ++j) {
+      const int col = n0 + (p.wn * GE::WJ + j) * 32 + (lane & 31);
+      if (col >= a.N) continue;
+      char* cb = c.base + int64_t(g) * 2 + int64_t(col) * a.G * 2;
+#pragma unroll
+      for (int i = 0; i < GE::WI; ++i)
+#pragma unroll
+        for (int qg = 0; qg < 4; ++qg)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int row = m0 + (p.wm * GE::WI + i) * 32 + qg * 8 + (lane >> 5) * 4 + e;
+            if (row < a.M) *reinterpret_cast<uint16_t*>(cb + int64_t(row) * c.rstride) = f2bf(acc[i][j][qg * 4 + e]);
+          }
+    }
+  } else if constexpr (OUT == OUT_PARTIAL) {
     // fp32 partial tile, straight from the accumulators: lane = one column,
     // 16 rows per MFMA tile; a wave store covers two 128-B row segments
     float* P = a.partial + (int64_t(sp) * a.G + g) * int64_t(a.M) * a.N;
     const int lane = p.lane;
 #pragma unroll
-    for (int i = 0; i < TMI; ++i)
+    for (int i = 0; i < GE::WI; ++i)
 #pragma unroll
-      for (int j = 0; j < TMJ; ++j) {
-        const int col = n0 + p.wn * WN + j * 32 + (lane & 31);
+      for (int j = 0; j < GE::WJ; ++j) {
+        const int col = n0 + (p.wn * GE::WJ + j) * 32 + (lane & 31);
         if (col >= a.N) continue;
 #pragma unroll
         for (int qg = 0; qg < 4; ++qg)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int row = m0 + p.wm * WM + i * 32 + qg * 8 + (lane >> 5) * 4 + e;
+            const int row = m0 + (p.wm * GE::WI + i) * 32 + qg * 8 + (lane >> 5) * 4 + e;
             if (row < a.M) P[int64_t(row) * a.N + col] = acc[i][j][qg * 4 + e];
           }
       }
   } else {
-    char* stage = reinterpret_cast<char*>(lds);
     barrier();  // every wave is done with the ring
-    stage_acc(stage, acc);
+    stage_acc<GE>(lds, acc);
     barrier_after_lds_writes();
     const GOut& c = a.c;
     char* cb = c.base + int64_t(g) * c.bstride;
-    const int wshift = 8 - c.log2l;
+    const int wshift = log2i(GE::BN) - c.log2l;
     const int ncol = (a.N - n0) >> c.log2l;  // valid destination columns per plane
-    write_tile(stage, c.log2l, [&](int r, int dc, const uint4& u) {
+    write_tile<GE>(lds, c.log2l, [&](int r, int dc, const uint4& u) {
       const int row = m0 + r;
       const int plane = dc >> wshift, col = dc & ((1 << wshift) - 1);
       if (row >= a.M || col >= ncol) return;
@@ -411,11 +494,11 @@ __device__ __forceinline__ void gemm_work(const GemmArgs& a, uint16_t* lds, int 
   }
 }
 
-template <bool AT, bool BT, bool SPLIT>
-__global__ __launch_bounds__(NT, 1) void butterfly_gemm(GemmArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint16_t lds[RING_ELEMS];
+template <class GE, bool AT, bool BT, int OUT>
+__global__ __launch_bounds__(GE::NTH, GE::PER_CU * GE::NW / 4) void butterfly_gemm(GemmArgs a) {
+  __shared__ __attribute__((aligned(1024))) char lds[GE::LDS];
   for (int v = blockIdx.x; v < a.vtiles; v += gridDim.x) {
-    gemm_work<AT, BT, SPLIT>(a, lds, v);
+    gemm_work<GE, AT, BT, OUT>(a, lds, v);
     barrier();  // the staging area is read before the next tile's loads refill the ring
   }
 }
@@ -449,6 +532,43 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* partial, int S
   }
 }
 
+// Feature order (B, s l) -> blocked rows (B, l, s): feature j l + b of a row is column j
+// of block b.  A thread reads 8 consecutive features (16 B) and writes 8 / l columns of
+// each block (one column of 8 of the 16 blocks), so a wave reads 1 KiB runs and writes
+// runs of 1 KiB / l per block.  HBM-bound: 4096 rows of 4 x 2752 take 27 us (90 MB, the
+// output stays in the Infinity Cache for the products that follow); a strided copy by
+// torch took 61.
+template <int L>
+__global__ __launch_bounds__(256) void to_blocks_kernel(const uint16_t* src, uint16_t* dst, int64_t chunks, int s) {
+  constexpr int U = 4;                        // chunks per thread
+  constexpr int C = L >= 8 ? 1 : 8 / L;       // columns per chunk and block
+  typedef uint16_t ColV __attribute__((ext_vector_type(C)));
+  const int cpr = s * L / 8;                  // chunks per row
+  const int64_t base = int64_t(blockIdx.x) * (256 * U) + threadIdx.x;
+  uint4 w[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (base + u * 256 < chunks) w[u] = *reinterpret_cast<const uint4*>(src + (base + u * 256) * 8);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = base + u * 256;
+    if (i >= chunks) continue;
+    const int64_t row = i / cpr;
+    const int f = int(i - row * cpr) * 8;     // first feature of the chunk
+    uint16_t* d = dst + row * (int64_t(s) * L) + int64_t(f % L) * s + f / L;
+    const uint32_t q[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+    for (int b = 0; b < 8 / C; ++b) {
+      ColV v;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int k = c * (8 / C) + b;
+        v[c] = uint16_t(q[k >> 1] >> (16 * (k & 1)));
+      }
+      *reinterpret_cast<ColV*>(d + int64_t(b) * s) = v;
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Host side: the six products as GemmArgs.
@@ -488,55 +608,95 @@ GOut make_out(void* base, int64_t bstride, int64_t rstride, int64_t rseg = UNSEG
 
 int cdiv(int64_t a, int64_t b) { return int((a + b - 1) / b); }
 
-void set_geometry(GemmArgs& a, int M, int N, int K, int G, int S) {
+typedef Geo<2, 4, 4, 2, 4> G256;  // 256 x 256 tiles, one workgroup per CU
+typedef Geo<2, 2, 2, 2, 4> G128;  // 128 x 128, two per CU
+typedef Geo<2, 2, 1, 1, 4> G64;   // 64 x 64, four per CU
+enum { T256 = 0, T128 = 1, T64 = 2 };
+
+// Tile size and number of K splits of a product, by a model of its time in ns on a
+// 256-CU part (a function of the shapes only, so the summation order, and with it the
+// result, does not depend on the device).  Large tiles read least per FLOP, small ones
+// fill the chip and have shorter prologues and epilogues.  Fitted to kernel times
+// (4096 tokens unless noted, us at 256 / 128 / 64-wide tiles): 4 x 512 x 512 products
+// 21.8 / 18.2 / 29.8, their weight gradients in 4 splits 29.8 / 18.6 / 29.8; 4 x 1024 x
+// 1024 44 / 58 / 96; 1000 tokens of 2 x 256 x 256 14.4 / 8.8 / 7.1; 8 tokens of 4 x 1024
+// x 1024 26 / 14 / 12.  (256 x 128 tiles, two workgroups per CU, were slower than 256 x
+// 256 wherever those fill the chip: 54 against 46 us on 16384 tokens of 2 x 512 x 1368.)
+struct GemmPlan {
+  int tile, S;
+};
+int64_t gemm_cost(int tile, int64_t M, int64_t N, int64_t G, int64_t K, int64_t S, bool wgrad) {
+  const int64_t side = tile == T256 ? 256 : tile == T128 ? 128 : 64;
+  const int64_t tiles = G * S * ((M + side - 1) / side) * ((N + side - 1) / side);
+  const int64_t rounds = (tiles + 255) / 256, k = (K + S - 1) / S;
+  int64_t t;
+  if (tile == T256) t = rounds * (8000 + k * (22 + 14 * std::min<int64_t>(tiles, 256) / 256));
+  else if (tile == T128) t = 4000 + rounds * (1000 + k * (wgrad ? 14 : rounds == 1 ? 9 : rounds == 2 ? 11 : 14));
+  else t = 4700 + std::max<int64_t>(tiles, 256) * (300 + k * 13 / 2) / 256;
+  // splits: the partials' write and read, and the reduction's launch
+  return S > 1 ? t + 4000 + S * G * M * N / 1400 : t;
+}
+// wgrad: a weight gradient, contracted over the tokens, whose K may be split (at least
+// 256 tokens per split).  no64: without the 64-wide tile.
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t G, int64_t K, bool wgrad, bool no64 = false) {
+  GemmPlan best{T256, 1};
+  int64_t best_cost = gemm_cost(T256, M, N, G, K, 1, wgrad);
+  for (int S = 1; S <= 64 && (S == 1 || (wgrad && K >= int64_t(S) * 256)); S *= 2)
+    for (int tile = T256; tile <= (no64 ? T128 : T64); ++tile) {
+      const int64_t c = gemm_cost(tile, M, N, G, K, S, wgrad);
+      if (c < best_cost) best = GemmPlan{tile, S}, best_cost = c;
+    }
+  return best;
+}
+
+void set_geometry(GemmArgs& a, int M, int N, int K, int G, GemmPlan plan) {
   a.M = M;
   a.N = N;
   a.K = K;
   a.G = G;
-  a.tiles_m = cdiv(M, BM);
-  a.tiles_n = cdiv(N, BN);
-  if (S > 1) {
-    a.kchunk = cdiv(cdiv(K, S), BK) * BK;
+  a.tile = plan.tile;
+  if (plan.S > 1) {
+    a.kchunk = cdiv(cdiv(K, plan.S), BK) * BK;
     a.S = cdiv(K, a.kchunk);
   } else {
     a.kchunk = cdiv(std::max(K, 1), BK) * BK;
     a.S = 1;
   }
-  a.vtiles = 8 * cdiv(int64_t(G) * a.S * a.tiles_m, 8) * a.tiles_n;
 }
 
-// Splits of a weight-gradient product (K = tokens), at least 1024 tokens per
-// split: the S that minimises a cost model of a 256-CU part in units of one
-// token of K per tile, rounds(S) (K/S + 576) + 768 [S > 1], where a round of
-// tiles carries a fixed cost of about 576 (prologue, epilogue, store burst) and
-// the fp32 partials' reduction pass about 768.  (6.89B at 4096 tokens: the
-// 64-tile products split 4 ways, the 176-tile ones run unsplit, one round of
-// K = 4096 instead of two of 2048 plus a reduction.)  A function of the shapes
-// only, so the summation order (and the result) does not depend on the device.
-int wgrad_splits(int M, int N, int G, int64_t K) {
-  const int64_t tiles = int64_t(G) * cdiv(M, BM) * cdiv(N, BN);
-  int best = 1;
-  int64_t best_cost = -1;
-  for (int S = 1; S <= 64 && (S == 1 || K >= int64_t(S) * 1024); S *= 2) {
-    const int64_t rounds = (tiles * S + 255) / 256;
-    const int64_t cost = rounds * ((K + S - 1) / S + 576) + (S > 1 ? 768 : 0);
-    if (best_cost < 0 || cost < best_cost) {
-      best = S;
-      best_cost = cost;
-    }
-  }
-  return best;
+template <class GE, bool AT, bool BT, int OUT>
+void launch_gemm_g(GemmArgs a, hipStream_t s) {
+  a.tiles_m = cdiv(a.M, GE::BM);
+  a.tiles_n = cdiv(a.N, GE::BN);
+  a.vtiles = OUT == OUT_FEATURES ? 8 * cdiv(int64_t(a.tiles_m) * a.tiles_n, 8) * a.G
+                                 : 8 * cdiv(int64_t(a.G) * a.S * a.tiles_m, 8) * a.tiles_n;
+  const int grid = std::min(a.vtiles, resident_grid(1 << 30) * GE::PER_CU);
+  hipLaunchKernelGGL((butterfly_gemm<GE, AT, BT, OUT>), dim3(grid), dim3(GE::NTH), 0, s, a);
 }
-
-template <bool AT, bool BT, bool SPLIT>
+template <bool AT, bool BT, int OUT>
 void launch_gemm_t(const GemmArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((butterfly_gemm<AT, BT, SPLIT>), dim3(resident_grid(a.vtiles)), dim3(NT), 0, s, a);
+  if (a.tile == T256) launch_gemm_g<G256, AT, BT, OUT>(a, s);
+  else if (a.tile == T128) launch_gemm_g<G128, AT, BT, OUT>(a, s);
+  else launch_gemm_g<G64, AT, BT, OUT>(a, s);
 }
 
 void launch_reduce(const GemmArgs& a, const GOut& c, hipStream_t s) {
   const int64_t total = int64_t(a.G) * a.M * (a.N / 8);
   const int blocks = int(std::min<int64_t>(std::max<int64_t>(1, (total + 255) / 256), 8192));
   hipLaunchKernelGGL(splitk_reduce, dim3(blocks), dim3(256), 0, s, a.partial, a.K > 0 ? a.S : 0, a.G, a.M, a.N, c);
+}
+
+void launch_to_blocks(const void* src, void* dst, int64_t rows, int l, int s, hipStream_t st) {
+  const int64_t chunks = rows * l * s / 8;
+  const dim3 grid(unsigned((chunks + 1023) / 1024)), block(256);
+  const auto* a = static_cast<const uint16_t*>(src);
+  auto* b = static_cast<uint16_t*>(dst);
+  switch (l) {
+    case 2: hipLaunchKernelGGL(to_blocks_kernel<2>, grid, block, 0, st, a, b, chunks, s); break;
+    case 4: hipLaunchKernelGGL(to_blocks_kernel<4>, grid, block, 0, st, a, b, chunks, s); break;
+    case 8: hipLaunchKernelGGL(to_blocks_kernel<8>, grid, block, 0, st, a, b, chunks, s); break;
+    default: hipLaunchKernelGGL(to_blocks_kernel<16>, grid, block, 0, st, a, b, chunks, s); break;
+  }
 }
 
 struct Dims {
@@ -552,15 +712,25 @@ Dims dims(const mmuon_butterfly_args& x) {
 
 }  // namespace
 
+// Weight gradients: dw2 (s x q per block) and dw1 (q x p), contracted over the tokens.
+GemmPlan dw2_plan(const Dims& d) { return gemm_plan(d.s, d.q, d.nb, d.B, true); }
+GemmPlan dw1_plan(const Dims& d) { return gemm_plan(d.q, d.p, d.nb, d.B, true); }
+
+size_t round256(size_t n) { return (n + 255) / 256 * 256; }
+
 size_t butterfly_workspace(const mmuon_butterfly_args& x) {
   const Dims d = dims(x);
   const size_t dt = size_t(d.nb) * d.B * d.q * 2;
-  const int s1 = wgrad_splits(d.s, d.q, d.nb, d.B), s4 = wgrad_splits(d.q, d.p, d.nb, d.B);
+  const int s1 = dw2_plan(d).S, s4 = dw1_plan(d).S;
   const size_t part = std::max(size_t(s1) * d.nb * d.s * d.q, size_t(s4) * d.nb * d.q * d.p) * 4;
-  return (dt + 255) / 256 * 256 + part;
+  return round256(dt) + part;
+}
+size_t butterfly_linear_workspace(const mmuon_butterfly_args& x) {
+  return butterfly_workspace(x) + (x.nblocks > 1 ? round256(size_t(x.nblocks) * x.tokens * x.s * 2) : 0);
 }
 
-int launch_butterfly_fwd(const mmuon_butterfly_args& x, hipStream_t st) {
+// features: out in feature order (B, s l) instead of (B, l, s)
+int launch_butterfly_fwd(const mmuon_butterfly_args& x, bool features, hipStream_t st) {
   const Dims d = dims(x);
   if (d.B == 0) return 0;
   const int64_t n = int64_t(d.nb) * d.p, ql = d.q / d.nb;
@@ -568,23 +738,32 @@ int launch_butterfly_fwd(const mmuon_butterfly_args& x, hipStream_t st) {
   f1.a = make_op(x.x, d.p * 2, n * 2, 2, int(d.B));
   f1.b = make_op(x.w1, int64_t(d.q) * d.p * 2, int64_t(d.p) * 2, 2, d.q);
   f1.c = make_out(x.out1, ql * 2, int64_t(d.q) * 2, UNSEG, 0, d.log2l, d.B * d.q * 2);
-  set_geometry(f1, int(d.B), d.q, d.p, d.nb, 1);
-  launch_gemm_t<false, false, false>(f1, st);
+  // (a 64-wide tile of 16 planes would write runs shorter than 16 B)
+  set_geometry(f1, int(d.B), d.q, d.p, d.nb, gemm_plan(d.B, d.q, d.nb, d.p, false, d.nb > 8));
+  launch_gemm_t<false, false, OUT_TILE>(f1, st);
   GemmArgs f2{};  // out[:, ll] = t[ll] . w2[ll]^T
   f2.a = make_op(x.out1, d.B * d.q * 2, int64_t(d.q) * 2, 2, int(d.B));
   f2.b = make_op(x.w2, int64_t(d.s) * d.q * 2, int64_t(d.q) * 2, 2, d.s);
   f2.c = make_out(x.out, int64_t(d.s) * 2, int64_t(d.nb) * d.s * 2);
-  set_geometry(f2, int(d.B), d.s, d.q, d.nb, 1);
-  launch_gemm_t<false, false, false>(f2, st);
+  set_geometry(f2, int(d.B), d.s, d.q, d.nb, gemm_plan(d.B, d.s, d.nb, d.q, false));
+  if (features && d.nb > 1) launch_gemm_t<false, false, OUT_FEATURES>(f2, st);
+  else launch_gemm_t<false, false, OUT_TILE>(f2, st);
   return 0;
 }
 
-int launch_butterfly_bwd(const mmuon_butterfly_args& x, hipStream_t st) {
+// features: dout in feature order (B, s l) instead of (B, l, s)
+int launch_butterfly_bwd(const mmuon_butterfly_args& xa, bool features, hipStream_t st) {
+  mmuon_butterfly_args x = xa;
   const Dims d = dims(x);
   const int64_t n = int64_t(d.nb) * d.p, ql = d.q / d.nb;
   char* ws = static_cast<char*>(x.workspace);
+  if (features && d.nb > 1 && d.B > 0) {
+    launch_to_blocks(x.dout, ws, d.B, d.nb, d.s, st);
+    x.dout = ws;
+    ws += round256(size_t(d.nb) * d.B * d.s * 2);
+  }
   void* dt = ws;
-  float* part = reinterpret_cast<float*>(ws + (size_t(d.nb) * d.B * d.q * 2 + 255) / 256 * 256);
+  float* part = reinterpret_cast<float*>(ws + round256(size_t(d.nb) * d.B * d.q * 2));
 
   // dw2[ll] = dout[:, ll]^T t[ll]  (K = tokens, split; unsplit: bf16 straight
   // from the tile)
@@ -593,17 +772,17 @@ int launch_butterfly_bwd(const mmuon_butterfly_args& x, hipStream_t st) {
   b1.b = make_op(x.out1, d.B * d.q * 2, 2, int64_t(d.q) * 2, d.q);
   b1.partial = part;
   b1.c = make_out(x.dw2, int64_t(d.s) * d.q * 2, int64_t(d.q) * 2);
-  set_geometry(b1, d.s, d.q, int(d.B), d.nb, wgrad_splits(d.s, d.q, d.nb, d.B));
+  set_geometry(b1, d.s, d.q, int(d.B), d.nb, dw2_plan(d));
   if (d.B > 0 && b1.S == 1) {
-    launch_gemm_t<true, true, false>(b1, st);
+    launch_gemm_t<true, true, OUT_TILE>(b1, st);
   } else {
-    if (d.B > 0) launch_gemm_t<true, true, true>(b1, st);
+    if (d.B > 0) launch_gemm_t<true, true, OUT_PARTIAL>(b1, st);
     launch_reduce(b1, b1.c, st);
   }
   if (d.B == 0) {
     GemmArgs b4{};
     b4.partial = part;
-    set_geometry(b4, d.q, d.p, 0, d.nb, 1);
+    set_geometry(b4, d.q, d.p, 0, d.nb, GemmPlan{T256, 1});
     launch_reduce(b4, make_out(x.dw1, int64_t(d.q) * d.p * 2, int64_t(d.p) * 2), st);
     return 0;
   }
@@ -612,8 +791,8 @@ int launch_butterfly_bwd(const mmuon_butterfly_args& x, hipStream_t st) {
   b2.a = make_op(x.dout, int64_t(d.s) * 2, int64_t(d.nb) * d.s * 2, 2, int(d.B));
   b2.b = make_op(x.w2, int64_t(d.s) * d.q * 2, 2, int64_t(d.q) * 2, d.q);
   b2.c = make_out(dt, d.B * d.q * 2, int64_t(d.q) * 2);
-  set_geometry(b2, int(d.B), d.q, d.s, d.nb, 1);
-  launch_gemm_t<false, true, false>(b2, st);
+  set_geometry(b2, int(d.B), d.q, d.s, d.nb, gemm_plan(d.B, d.q, d.nb, d.s, false));
+  launch_gemm_t<false, true, OUT_TILE>(b2, st);
 
   // dx[:, kk] = sum over (ll, j) of dt[ll][:, kk q/l + j] w1[kk][j l + ll]: K in
   // segments of q/l, one per plane ll (the unriffle folded into the addressing)
@@ -621,8 +800,8 @@ int launch_butterfly_bwd(const mmuon_butterfly_args& x, hipStream_t st) {
   b3.a = make_op(dt, ql * 2, int64_t(d.q) * 2, 2, int(d.B), UNSEG, 0, ql, d.B * d.q * 2);
   b3.b = make_op(x.w1, int64_t(d.q) * d.p * 2, 2, int64_t(d.nb) * d.p * 2, d.p, UNSEG, 0, ql, int64_t(d.p) * 2);
   b3.c = make_out(x.dx, int64_t(d.p) * 2, n * 2);
-  set_geometry(b3, int(d.B), d.p, d.q, d.nb, 1);
-  launch_gemm_t<false, true, false>(b3, st);
+  set_geometry(b3, int(d.B), d.p, d.q, d.nb, gemm_plan(d.B, d.p, d.nb, d.q, false));
+  launch_gemm_t<false, true, OUT_TILE>(b3, st);
 
   // dw1[kk] with rows in (ll, j) order: row ll q/l + j of the product is
   // dw1 row j l + ll (the reduction writes it there)
@@ -631,11 +810,11 @@ int launch_butterfly_bwd(const mmuon_butterfly_args& x, hipStream_t st) {
   b4.b = make_op(x.x, int64_t(d.p) * 2, 2, n * 2, d.p);
   b4.partial = part;
   b4.c = make_out(x.dw1, int64_t(d.q) * d.p * 2, int64_t(d.nb) * d.p * 2, ql, int64_t(d.p) * 2);
-  set_geometry(b4, d.q, d.p, int(d.B), d.nb, wgrad_splits(d.q, d.p, d.nb, d.B));
+  set_geometry(b4, d.q, d.p, int(d.B), d.nb, dw1_plan(d));
   if (b4.S == 1) {
-    launch_gemm_t<true, true, false>(b4, st);
+    launch_gemm_t<true, true, OUT_TILE>(b4, st);
   } else {
-    launch_gemm_t<true, true, true>(b4, st);
+    launch_gemm_t<true, true, OUT_PARTIAL>(b4, st);
     launch_reduce(b4, b4.c, st);
   }
   return 0;

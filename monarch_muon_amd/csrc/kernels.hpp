@@ -86,9 +86,11 @@ int set_error(int code, const char* msg);
 int launch_status(const char* what);
 
 // Monarch butterfly multiply -------------------------------------------------------
+// (features / _linear_: out and dout in feature order)
 size_t butterfly_workspace(const mmuon_butterfly_args& a);
-int launch_butterfly_fwd(const mmuon_butterfly_args& a, hipStream_t s);
-int launch_butterfly_bwd(const mmuon_butterfly_args& a, hipStream_t s);
+size_t butterfly_linear_workspace(const mmuon_butterfly_args& a);
+int launch_butterfly_fwd(const mmuon_butterfly_args& a, bool features, hipStream_t s);
+int launch_butterfly_bwd(const mmuon_butterfly_args& a, bool features, hipStream_t s);
 
 // Gradient-clipping coefficient of a launch (gscale: device pointer, or null
 // when not clipping), read once per thread: the per-element form would test

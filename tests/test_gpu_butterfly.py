@@ -75,6 +75,45 @@ def test_forward_and_backward_match_oracle(case):
         assert v <= TOL, (k, v)
 
 
+# one case for each tile size (64-, 128- and 256-wide) beside those above, an unsplit and a split weight gradient at
+# each, row counts one past and one short of a tile, and rows that are no multiple of the interleaving pass's stride
+LINEAR_CASES = CASES + [(1, 4, 1024, 1024, 2752), (65, 2, 64, 136, 72), (127, 2, 192, 192, 200), (4096, 4, 512, 512, 512),
+                        (2049, 2, 512, 1368, 520), (8191, 4, 256, 256, 264), (3001, 4, 1024, 1024, 1024),
+                        (0, 2, 256, 256, 256)]
+
+
+@pytest.mark.parametrize("case", LINEAR_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_layer_form_equals_the_blocked_pair(case):
+    """butterfly_blk (feature-order output and gradient) against the blocked op pair, bit for bit: the same products
+    with the same summation order, their results stored elsewhere.  The pair against the oracle's products in fp32."""
+    print("butterfly case", case, flush=True)
+    tokens, nb, q, p, s = case
+    x, w1, w2, dout = gpu(*make(*case, seed=3))
+    out, out1 = butterfly_blk_op(x, w1, w2)
+    grads = butterfly_blk_bwd_op(x, w1, w2, out1, dout)
+    xg, w1g, w2g = (t.clone().requires_grad_() for t in (x, w1, w2))
+    y = butterfly_blk(xg, w1g, w2g)
+    dy = dout.transpose(1, 2).reshape(tokens, s * nb)
+    got = torch.autograd.grad(y, (xg, w1g, w2g), dy)
+    torch.cuda.synchronize()
+    assert torch.equal(y, out.transpose(1, 2).reshape(tokens, s * nb))
+    for u, v in zip(got, grads):
+        assert torch.equal(u, v)
+    if tokens:
+        ref_out, ref_out1 = bf.butterfly_fwd(x, w1, w2)
+        ref = (ref_out, ref_out1) + bf.butterfly_bwd(x, w1, w2, out1, dout)
+        for u, v in zip((out, out1) + tuple(grads), ref):
+            assert rel(u, v) <= TOL
+
+
+def test_gradient_through_the_intermediate_alone_is_zero():
+    """out1 carries no gradient of its own; asking for one through it alone gives zeros."""
+    x, w1, w2, _ = gpu(*make(64, 2, 64, 64, 64))
+    x.requires_grad_()
+    (g,) = torch.autograd.grad(butterfly_blk_op(x, w1, w2)[1].sum(), (x,))
+    assert not g.any()
+
+
 def test_zero_tokens():
     x, w1, w2, dout = make(0, 4, 256, 256, 256)
     xg, w1g, w2g, dg = gpu(x, w1, w2, dout)
