@@ -1,8 +1,9 @@
 """Build ``libmmuon.so`` (gfx950) in-tree with hipcc.
 
 ``python -m monarch_muon_amd.build`` compiles every ``csrc/*.hip`` to an object
-in parallel and links the shared library next to this file.  hipcc
-cross-compiles for gfx950 without a GPU.  ``build_probe()`` builds the
+in parallel and links the shared library next to this file, and beside it
+``libmmuon_torch.so``, the layer's native torch operator (``csrc/torch_ops.cpp``,
+host code only).  hipcc cross-compiles for gfx950 without a GPU.  ``build_probe()`` builds the
 bench-only HBM streaming probe (``bench_probe.hip`` beside ``bench.py``) into a
 library of its own, apart from the optimizer's.
 """
@@ -18,6 +19,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libmmuon.so"
+TORCH_LIB = HERE / "libmmuon_torch.so"
 ARCH = "gfx950"
 
 CFLAGS = [
@@ -47,14 +49,32 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{msg}")
 
 
+def _build_torch_ops() -> None:
+    import torch
+    inc = Path(torch.__file__).resolve().parent
+    rocm = Path(_hipcc()).resolve().parent.parent
+    tmp = TORCH_LIB.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", str(inc / "include"), "-isystem", str(inc / "include/torch/csrc/api/include"),
+           "-isystem", str(rocm / "include"), "-isystem", "/opt/rocm/include", str(CSRC / "torch_ops.cpp"),
+           "-o", str(tmp), f"-L{inc / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"torch_ops.cpp failed:\n{r.stdout}{r.stderr}")
+    os.replace(tmp, TORCH_LIB)
+
+
 def build(verbose: bool = True) -> Path:
     srcs = sorted(CSRC.glob("*.hip"))
     objdir = HERE / "_build"
     objdir.mkdir(exist_ok=True)
     objs = [objdir / (s.stem + ".o") for s in srcs]
     jobs = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", os.cpu_count() or 4))))
-    with cf.ThreadPoolExecutor(jobs) as ex:
+    with cf.ThreadPoolExecutor(jobs + 1) as ex:
+        ops = ex.submit(_build_torch_ops)
         list(ex.map(_compile, srcs, objs))
+        ops.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -20,6 +20,7 @@ the reference's models satisfies.  Other inputs raise; there is no fallback.
 from __future__ import annotations
 
 import ctypes as C
+from pathlib import Path
 
 import torch
 
@@ -47,49 +48,44 @@ def _args(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> _abi.Butterfl
     return a
 
 
-def _fwd(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, features: bool) -> tuple[torch.Tensor, torch.Tensor]:
-    """(out, out1): ``out`` blocked (B, l, s), or with ``features`` in feature order (B, s l)."""
+def _fwd(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     x2, w1, w2 = x2.contiguous(), w1.contiguous(), w2.contiguous()
     a = _args(x2, w1, w2)
     B = x2.shape[0]
     l, s, r = w2.shape
-    out = torch.empty((B, s * l) if features else (B, l, s), device=x2.device, dtype=x2.dtype)
+    out_blk = torch.empty(B, l, s, device=x2.device, dtype=x2.dtype)
     out1 = torch.empty(l, B, r, device=x2.device, dtype=x2.dtype)
-    a.out, a.out1 = out.data_ptr(), out1.data_ptr()
-    fn = _abi.lib().mmuon_butterfly_linear_fwd if features else _abi.lib().mmuon_butterfly_fwd
-    _abi.check(fn(C.byref(a), _abi.stream_handle(x2.device)), "mmuon_butterfly_fwd")
-    return out, out1
+    a.out, a.out1 = out_blk.data_ptr(), out1.data_ptr()
+    _abi.check(_abi.lib().mmuon_butterfly_fwd(C.byref(a), _abi.stream_handle(x2.device)), "mmuon_butterfly_fwd")
+    return out_blk, out1
 
 
-def _bwd(x2, w1, w2, out1, dout, features: bool):
-    """(dx, dw1, dw2) from ``dout`` in the layout of ``_fwd``'s ``out``."""
+def _bwd(x2, w1, w2, out1, dout_blk):
     x2, w1, w2 = x2.contiguous(), w1.contiguous(), w2.contiguous()
-    out1, dout = out1.contiguous(), dout.contiguous()
+    out1, dout_blk = out1.contiguous(), dout_blk.contiguous()
     a = _args(x2, w1, w2)
     B = x2.shape[0]
     l, s, r = w2.shape
-    if tuple(out1.shape) != (l, B, r) or tuple(dout.shape) != ((B, s * l) if features else (B, l, s)):
-        raise ValueError(f"out1 {tuple(out1.shape)} / dout {tuple(dout.shape)} do not match the forward")
-    if out1.dtype != torch.bfloat16 or dout.dtype != torch.bfloat16:
+    if tuple(out1.shape) != (l, B, r) or tuple(dout_blk.shape) != (B, l, s):
+        raise ValueError(f"out1 {tuple(out1.shape)} / dout {tuple(dout_blk.shape)} do not match the forward")
+    if out1.dtype != torch.bfloat16 or dout_blk.dtype != torch.bfloat16:
         raise TypeError("out1 and dout must be bfloat16")
-    _abi._require_cuda(out1, dout)
+    _abi._require_cuda(out1, dout_blk)
     dx = torch.empty_like(x2)
     dw1 = torch.empty_like(w1)
     dw2 = torch.empty_like(w2)
-    a.out1, a.dout, a.dx, a.dw1, a.dw2 = (out1.data_ptr(), dout.data_ptr(), dx.data_ptr(),
+    a.out1, a.dout, a.dx, a.dw1, a.dw2 = (out1.data_ptr(), dout_blk.data_ptr(), dx.data_ptr(),
                                           dw1.data_ptr(), dw2.data_ptr())
-    lib = _abi.lib()
-    nbytes = lib.mmuon_butterfly_linear_workspace(C.byref(a)) if features else lib.mmuon_butterfly_workspace(C.byref(a))
+    nbytes = _abi.lib().mmuon_butterfly_workspace(C.byref(a))
     ws = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=x2.device)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    fn = lib.mmuon_butterfly_linear_bwd if features else lib.mmuon_butterfly_bwd
-    _abi.check(fn(C.byref(a), _abi.stream_handle(x2.device)), "mmuon_butterfly_bwd")
+    _abi.check(_abi.lib().mmuon_butterfly_bwd(C.byref(a), _abi.stream_handle(x2.device)), "mmuon_butterfly_bwd")
     return dx, dw1, dw2
 
 
 @torch.library.custom_op("mmuon::butterfly_blk", mutates_args=())
 def butterfly_blk_op(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    return _fwd(x2, w1, w2, False)
+    return _fwd(x2, w1, w2)
 
 
 @butterfly_blk_op.register_fake
@@ -102,27 +98,7 @@ def _(x2, w1, w2):
 @torch.library.custom_op("mmuon::butterfly_blk_bwd", mutates_args=())
 def butterfly_blk_bwd_op(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, out1: torch.Tensor,
                          dout_blk: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    return _bwd(x2, w1, w2, out1, dout_blk, False)
-
-
-# The layer's own form of the pair: output and its gradient in feature order, (B, s l) with feature
-# j l + ll the column j of block ll, so no interleaving pass follows the forward's products.
-@torch.library.custom_op("mmuon::butterfly_linear", mutates_args=())
-def _linear_op(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    return _fwd(x2, w1, w2, True)
-
-
-@_linear_op.register_fake
-def _(x2, w1, w2):
-    B = x2.shape[0]
-    l, s, r = w2.shape
-    return x2.new_empty(B, s * l), x2.new_empty(l, B, r)
-
-
-@torch.library.custom_op("mmuon::butterfly_linear_bwd", mutates_args=())
-def _linear_bwd_op(x2: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, out1: torch.Tensor,
-                   dout: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    return _bwd(x2, w1, w2, out1, dout, True)
+    return _bwd(x2, w1, w2, out1, dout_blk)
 
 
 def _bwd_fake(x2, w1, w2, out1, dout):
@@ -130,28 +106,56 @@ def _bwd_fake(x2, w1, w2, out1, dout):
 
 
 butterfly_blk_bwd_op.register_fake(_bwd_fake)
-_linear_bwd_op.register_fake(_bwd_fake)
 
 
-def _register_autograd(op, bwd_op):
-    def setup_context(ctx, inputs, output):
-        x2, w1, w2 = inputs
-        ctx.save_for_backward(x2, w1, w2, output[1])
-        # out1 is saved for the backward and has no gradient of its own: no zeros are made for it
-        ctx.set_materialize_grads(False)
-        ctx.out_shape = output[0].shape
-
-    def backward(ctx, dout, dout1_unused):
-        x2, w1, w2, out1 = ctx.saved_tensors
-        if dout is None:
-            dout = x2.new_zeros(ctx.out_shape)
-        return bwd_op(x2, w1, w2, out1, dout.contiguous())
-
-    op.register_autograd(backward, setup_context=setup_context)
+def _setup_context(ctx, inputs, output):
+    x2, w1, w2 = inputs
+    ctx.save_for_backward(x2, w1, w2, output[1])
+    # out1 is saved for the backward and has no gradient of its own: no zeros are made for it
+    ctx.set_materialize_grads(False)
+    ctx.out_shape = output[0].shape
 
 
-_register_autograd(butterfly_blk_op, butterfly_blk_bwd_op)
-_register_autograd(_linear_op, _linear_bwd_op)
+def _backward(ctx, dout_blk, dout1_unused):
+    x2, w1, w2, out1 = ctx.saved_tensors
+    if dout_blk is None:
+        dout_blk = x2.new_zeros(ctx.out_shape)
+    return butterfly_blk_bwd_op(x2, w1, w2, out1, dout_blk.contiguous())
+
+
+butterfly_blk_op.register_autograd(_backward, setup_context=_setup_context)
+
+
+# The layer's own form of the pair, ``mmuon::butterfly_linear`` and ``mmuon::butterfly_linear_bwd``
+# (csrc/torch_ops.cpp, autograd included): output and its gradient in feature order, (B, s l) with
+# feature j l + ll the column j of block ll, so no interleaving pass follows the products.
+_TORCH_LIB = Path(__file__).resolve().parent / "libmmuon_torch.so"
+_BOUND = ("mmuon_butterfly_linear_fwd", "mmuon_butterfly_linear_bwd", "mmuon_butterfly_linear_workspace",
+          "mmuon_last_error")
+
+
+def _load_linear():
+    """The native operator, bound to the library ``_abi`` loads; raises where either is missing."""
+    lib = _abi.lib()
+    if not _TORCH_LIB.exists():
+        raise RuntimeError(f"{_TORCH_LIB} is missing: build it with `python -m monarch_muon_amd.build`")
+    torch.ops.load_library(str(_TORCH_LIB))
+    C.CDLL(str(_TORCH_LIB)).mmuon_torch_bind(*(C.cast(getattr(lib, name), C.c_void_p) for name in _BOUND))
+
+    @torch.library.register_fake("mmuon::butterfly_linear")
+    def _(x2, w1, w2):
+        B = x2.shape[0]
+        l, s, r = w2.shape
+        return x2.new_empty(B, s * l), x2.new_empty(l, B, r)
+
+    torch.library.register_fake("mmuon::butterfly_linear_bwd", _bwd_fake)
+    return torch.ops.mmuon.butterfly_linear.default
+
+
+try:
+    _linear_op = _load_linear()
+except (RuntimeError, OSError) as e:   # not built: the first call raises
+    _linear_op, _linear_error = None, e
 
 
 def butterfly_blk(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> torch.Tensor:
@@ -159,6 +163,10 @@ def butterfly_blk(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> torch.
     if torch.is_autocast_enabled():
         dt = torch.get_autocast_dtype("cuda")
         x, w1, w2 = x.to(dt), w1.to(dt), w2.to(dt)
+    if _linear_op is None:
+        raise RuntimeError(str(_linear_error))
+    if x.dim() == 2:
+        return _linear_op(x, w1, w2)[0]
     batch_shape, n = x.shape[:-1], x.shape[-1]
     out, _ = _linear_op(x.reshape(-1, n), w1, w2)
     return out.view(*batch_shape, out.shape[1])

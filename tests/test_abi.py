@@ -151,3 +151,19 @@ def test_hbm_probe_validates_before_launching():
     assert lib.probe_hbm_stream(0, 4096, 4096, 4096 * 64, 0, 65, None) == -1
     assert lib.probe_hbm_stream(3, 4096, 4096, 16384 * 16, 0, 17, None) == -1
     assert b"read probe" in lib.probe_last_error()
+
+
+def test_layer_operator_shapes_and_refusals():
+    """The layer's native operator on meta tensors (forward and backward shapes) and what it refuses."""
+    import pytest
+    import torch
+
+    from monarch_muon_amd import butterfly_blk
+    x, w1, w2 = torch.randn(4, 64).bfloat16(), torch.randn(2, 32, 32).bfloat16(), torch.randn(2, 40, 32).bfloat16()
+    with pytest.raises(RuntimeError, match="ROCm GPU"):
+        butterfly_blk(x, w1, w2)
+    a = [t.to("meta").requires_grad_() for t in (x, w1, w2)]
+    for lead in ((4,), (2, 2), ()):
+        y = butterfly_blk(a[0].reshape(-1)[:64 * max(1, 4 if lead else 1)].reshape(*lead, 64), a[1], a[2])
+        assert y.shape == (*lead, 80)
+        assert [g.shape for g in torch.autograd.grad(y.sum(), a)] == [t.shape for t in a]

@@ -106,6 +106,30 @@ def test_layer_form_equals_the_blocked_pair(case):
             assert rel(u, v) <= TOL
 
 
+@pytest.mark.parametrize("how", ["compile", "saved_hooks", "expanded_grad", "second_order"])
+def test_layer_operator_under_torch(how):
+    """The native operator traced by torch.compile, with saved-tensor hooks and with a gradient that is no dense
+    tensor, against the plain call; a second derivative is refused."""
+    x, w1, w2, _ = gpu(*make(96, 2, 64, 64, 72, seed=4))
+    a, b = ([t.clone().requires_grad_() for t in (x, w1, w2)] for _ in range(2))
+    y = butterfly_blk(*a)
+    if how == "second_order":
+        (g, *_) = torch.autograd.grad(y.float().pow(2).sum(), a, create_graph=True)
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            torch.autograd.grad(g.float().sum(), a)
+        return
+    want = torch.autograd.grad(y, a, torch.ones_like(y))
+    if how == "compile":
+        z = torch.compile(lambda *t: butterfly_blk(*t), backend="aot_eager", fullgraph=True)(*b)
+    elif how == "saved_hooks":
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(DEV)):
+            z = butterfly_blk(*b)
+    else:
+        z = butterfly_blk(*b)
+    got = torch.autograd.grad(z.sum(), b)   # an expanded gradient
+    assert torch.equal(y, z) and all(torch.equal(u, v) for u, v in zip(got, want))
+
+
 def test_gradient_through_the_intermediate_alone_is_zero():
     """out1 carries no gradient of its own; asking for one through it alone gives zeros."""
     x, w1, w2, _ = gpu(*make(64, 2, 64, 64, 64))
