@@ -66,7 +66,7 @@ typedef struct mmuon_block_fp8 {
    element (i, j) of an R-row matrix at (j / 32) * R * 32 + i * 32 + j % 32. */
 typedef struct mmuon_ns_layout_t {
   int32_t m, n;        /* Newton-Schulz orientation: m = min(r,c), n = max(r,c) */
-  int32_t mp, np_;     /* padded m, n (multiples of the kernels' tiles)          */
+  int32_t mp, np_;     /* padded m, n                                            */
   int32_t nparts;      /* partial sums of squares per block                      */
   int32_t ns_dtype;    /* MMUON_BF16 or MMUON_F32                                */
   int64_t x_bytes;     /* one X stack  [N] x (mp x np_)                           */
@@ -133,8 +133,8 @@ int mmuon_fp8_momentum_pack(const mmuon_group* g, float momentum, int32_t have_s
      param <- param + alpha * cast(X) (un-transposed), alpha = -lr*sqrt(r/c)
    coeffs = {a, b, c}.  The launches are the ops of mmuon_ns_plan(g->rows,
    g->cols, g->ns_dtype, iters, flags): the three-product chain (X ping-pongs
-   between x0 and x1), or for bf16 groups with np_ >= 2 mp and iters == 5 the
-   Gram form (see mmuon_ns_plan).  flags: MMUON_NS_NO_APPLY leaves the final X
+   between x0 and x1), or for bf16 groups with n >= 2 m, both rounded up to
+   multiples of 256, and iters == 5 the Gram form (see mmuon_ns_plan).  flags: MMUON_NS_NO_APPLY leaves the final X
    in the workspace stack named by the plan's last op (standard chain: x0 when
    iters is even, x1 otherwise; Gram form: x0) and does not touch params;
    MMUON_NS_STANDARD selects the three-product chain for every group;
@@ -191,7 +191,7 @@ typedef struct mmuon_ns_op {
 /* The launch plan of mmuon_newton_schulz_apply for a group of (rows x cols)
    blocks: writes up to max_ops ops (none when ops is NULL) and returns their
    number, or a negative error code.  Three-product chain: SYRK, POLY, PX per
-   iteration.  Gram form (ns_dtype BF16, np_ >= 2 mp, iters == 5, no
+   iteration.  Gram form (ns_dtype BF16, n >= 2 m in multiples of 256, iters == 5, no
    MMUON_NS_STANDARD): X_k = Q_k X_0 with Q_k a polynomial in A_0 = X_0 X_0^T, so
      P_k = a I + b A_k + c A_k^2, Q_{k+1} = P_k Q_k, A_{k+1} = P_k (P_k A_k)
    run on m x m matrices; X is rebuilt once (X_3 = Q_3 X_0) and the last two

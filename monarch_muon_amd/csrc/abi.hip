@@ -61,6 +61,13 @@ struct Geometry {
   bool transposed;
 };
 
+// Blocks whose bf16 Newton-Schulz takes the Gram form: the long side at least twice
+// the short one, both in whole 256-wide tiles (the unit the two forms' costs were
+// compared in; the choice does not follow the finer padding of the stacks).
+bool gram_sides(int m, int n, int ns_dtype) {
+  return ns_dtype == MMUON_BF16 && roundup(n, 256) >= 2 * roundup(m, 256);
+}
+
 int geometry(int rows, int cols, int ns_dtype, Geometry& g) {
   if (rows <= 0 || cols <= 0) return fail(MMUON_EINVAL, "block shape must be positive (%d x %d)", rows, cols);
   if (ns_dtype != MMUON_BF16 && ns_dtype != MMUON_F32)
@@ -68,8 +75,9 @@ int geometry(int rows, int cols, int ns_dtype, Geometry& g) {
   g.transposed = rows > cols;
   g.m = std::min(rows, cols);
   g.n = std::max(rows, cols);
-  const int tm = mmuon::ns_tile_m(ns_dtype), tn = mmuon::ns_tile_n(ns_dtype);
-  const int64_t mp = roundup(g.m, tm), np_ = roundup(g.n, std::max(tn, 64));
+  const int64_t mp = roundup(g.m, mmuon::ns_pad(ns_dtype, g.m));
+  int64_t np_ = roundup(g.n, mmuon::ns_pad(ns_dtype, g.n));
+  if (gram_sides(g.m, g.n, ns_dtype)) np_ = std::max(np_, 2 * mp);  // two m x m stacks fit in one X stack
   if (mp > (1 << 15) || np_ > (1 << 15)) return fail(MMUON_ERANGE, "block side beyond 32768 (%d x %d)", rows, cols);
   g.mp = int(mp);
   g.np_ = int(np_);
@@ -207,8 +215,8 @@ namespace {
 // caller (per-launch timing, the stage tests) and mmuon_ns_run_op runs one op.
 //
 // Standard chain, per iteration: A = X X^T; P = a I + b A + c A A; X = P X
-// (the a X term on P's diagonal).  Gram form (bf16 groups with n >= 2m after
-// padding, 5 iterations): every X_k = Q_k X_0 with Q_k a polynomial in the
+// (the a X term on P's diagonal).  Gram form (bf16 groups with n >= 2m in whole
+// 256-wide tiles, 5 iterations): every X_k = Q_k X_0 with Q_k a polynomial in the
 // first Gram matrix A_0, so the iterations can run on m x m matrices:
 //   P_k = a I + b A_k + c A_k^2,  Q_{k+1} = P_k Q_k,  A_{k+1} = P_k (P_k A_k)
 // (all symmetric and commuting: products of polynomials in A_0).  This
@@ -237,8 +245,7 @@ bool overlaps(int u, int v) {
 }
 
 bool gram_eligible(const Geometry& geo, int ns_dtype, int iters, int flags) {
-  return ns_dtype == MMUON_BF16 && !(flags & MMUON_NS_STANDARD) && iters == 5 &&
-         int64_t(geo.np_) >= 2 * int64_t(geo.mp);
+  return !(flags & MMUON_NS_STANDARD) && iters == 5 && gram_sides(geo.m, geo.n, ns_dtype);
 }
 
 void build_plan(const Geometry& geo, int ns_dtype, int iters, int flags, std::vector<mmuon_ns_op>& ops) {

@@ -46,8 +46,7 @@ struct NsArgs {
 };
 
 // geometry helpers (tile sizes of the kernels)
-int ns_tile_m(int ns_dtype);
-int ns_tile_n(int ns_dtype);
+int ns_pad(int ns_dtype, int side);  // what a block side is padded to a multiple of
 int ns_tile_k(int ns_dtype);
 int launch_ns_stage(const NsArgs& a, int stage, int ns_dtype, int param_dtype, hipStream_t s);
 

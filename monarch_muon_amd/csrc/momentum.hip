@@ -25,7 +25,7 @@ constexpr int PACK_ELEMS = PACK_NT * 8 * PACK_ITERS;  // X elements per workgrou
 
 // rows <= cols: X[b][i][j] = buf[b][i][j], 8 elements per thread.
 // fp32 X: the padded [mp][np] extent is walked in row-major order.
-// bf16 X (32-column panels; mp, np multiples of 256): a workgroup owns 32 rows x
+// bf16 X (32-column panels; mp, np multiples of 64): a workgroup owns 32 rows x
 // 256 columns, and per iteration a wave covers 8 rows x 64 columns, so every
 // wave reads whole 128-B lines of the momentum and gradient rows and writes two
 // contiguous 512-B panel runs.
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(PACK_NT) void pack_rows_kernel(PackArgs a) {
   auto* buf = reinterpret_cast<typename TB::storage*>(ref.buf);
   auto* x = reinterpret_cast<typename TX::storage*>(a.x) + int64_t(b) * a.mp * a.np;
   const int64_t total = int64_t(a.mp) * a.np;
-  const int tiles_j = a.np / 256;
+  const int tiles_j = (a.np + 255) / 256;  // the last one partial when np % 256 != 0
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const GradClip clip = grad_clip(a.gscale);
   float ss = 0.f;
@@ -81,6 +81,7 @@ __global__ __launch_bounds__(PACK_NT) void pack_rows_kernel(PackArgs a) {
     if constexpr (PANELS) {
       i = (blockIdx.x / tiles_j) * 32 + wave * 8 + (lane >> 3);
       j = (blockIdx.x % tiles_j) * 256 + it * 64 + (lane & 7) * 8;
+      if (j >= a.np) break;  // uniform: np is a multiple of 64
     } else {
       const int64_t e = int64_t(blockIdx.x) * PACK_ELEMS + (int64_t(it) * PACK_NT + threadIdx.x) * 8;
       if (e >= total) break;
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(PACK_NT) void pack_rows_kernel(PackArgs a) {
 // X writes are one contiguous 16 KiB run.
 constexpr int PCOL_ROWS = 32;   // buf rows per workgroup
 constexpr int PCOL_COLS = 256;  // buf columns per workgroup (= PACK_NT)
-static_assert(PCOL_COLS == PACK_NT, "one X row per thread in phase 2");
+static_assert(PCOL_COLS == PACK_NT && PACK_ELEMS == 32 * 256, "one X row per thread in phase 2");
 template <class TG, class TB, class TX>
 __global__ __launch_bounds__(PACK_NT) void pack_cols_kernel(PackArgs a) {
   __shared__ float tile[PCOL_ROWS][PCOL_COLS + 4];
@@ -210,8 +211,7 @@ __global__ __launch_bounds__(PACK_NT) void pack_cols_kernel(PackArgs a) {
 
 int pack_nparts(int mp, int np_, bool transposed) {
   if (transposed) return ((mp + PCOL_COLS - 1) / PCOL_COLS) * (np_ / PCOL_ROWS);
-  const int64_t total = int64_t(mp) * np_;
-  return int((total + PACK_ELEMS - 1) / PACK_ELEMS);
+  return (mp / 32) * ((np_ + 255) / 256);  // workgroups of 32 x 256 (fp32 X: of as many elements in a row)
 }
 
 template <class TG, class TB, class TX>

@@ -40,6 +40,8 @@ namespace {
 // Tiles of a symmetric m x m product: BM-row band ti, BN-column band tc with
 // tc >= R ti, R = BM / BN (the upper triangle and the diagonal blocks), ti-major.
 constexpr int R_SYM = BM / BN;
+// 256-wide tiles over an extent (a multiple of 64), the last one possibly partial
+__host__ __device__ __forceinline__ int tiles_of(int extent) { return (extent + BM - 1) / BM; }
 __device__ __forceinline__ void sym_tile(int t, int nc, int& ti, int& tc) {
   int i = 0;
   while (t >= nc - R_SYM * i) {
@@ -101,6 +103,10 @@ struct Pipe {
   const uint16_t* csrc_t;
   int thr_r, thr_c;        // OP_SPLIT: slices kt < thr are T
   uint32_t pstride_b;      // bytes per panel (rows * 32 * 2; a block is below 2^31 bytes)
+  // this wave's loads, byte offsets within a slice's source: K form, its two 16-row
+  // chunks; T form, its panel.  Beyond the stack's extent (a partial tile) the last
+  // chunk or panel is loaded again; it feeds outputs that are not stored.
+  uint32_t rk[2], ck[2], rt, ct;
   int KT;
   int wave, lane, wm, wn;
   uint16_t* lds;  // ring slot s at lds + s*SLOT: row-operand slice, then column-operand slice
@@ -139,11 +145,10 @@ struct Pipe {
     // 32-bit byte offsets from the operand's base
     const uint32_t ks = uint32_t(src_kt);
     if (t)
-      dma16(reinterpret_cast<const char*>(srct) + (ks * (BK * PANEL * 2) + uint32_t(wave) * pstride_b + q * 16 * PANEL * 2),
+      dma16(reinterpret_cast<const char*>(srct) + (ks * (BK * PANEL * 2) + (Q < 2 ? rt : ct) + q * 16 * PANEL * 2),
             uint32_t(lane) << 4, dst);
     else
-      dma16(reinterpret_cast<const char*>(srck) + (ks * pstride_b + uint32_t(2 * wave + q) * (16 * PANEL * 2)), k_loff,
-            dst);
+      dma16(reinterpret_cast<const char*>(srck) + (ks * pstride_b + (Q < 2 ? rk[q] : ck[q])), k_loff, dst);
   }
   __device__ __forceinline__ void issue(int src_kt, int slot_kt) const {
     issue_one<0>(src_kt, slot_kt);
@@ -377,13 +382,17 @@ __device__ __forceinline__ WavePlan diag_plan(int wave) {
 // w + 4): a K slice that crosses a window's identity columns (POLY) then
 // gives each SIMD one wave of identity work beside its other wave's MFMAs,
 // instead of both of one SIMD's waves while the others wait at the barrier.
-__device__ __forceinline__ WavePlan full_plan(int wave) { return {wave & 1, wave >> 1, MASK_FULL}; }
+// A tile with at most 128 valid rows keeps only its upper windows busy: there the
+// four busy waves go to four SIMDs instead of two.
+__device__ __forceinline__ WavePlan full_plan(int wave, int rows) {
+  return rows > WM ? WavePlan{wave & 1, wave >> 1, MASK_FULL} : WavePlan{wave >> 2, wave & 3, MASK_FULL};
+}
 
 template <int RK, int CK, int IDENT, int MASK, bool SHARED>
 __device__ __forceinline__ void mainloop_run(const uint16_t* rsrc_k, const uint16_t* rsrc_t, int thr_r,
                                              const uint16_t* csrc_k, const uint16_t* csrc_t, int thr_c,
                                              int64_t pstride, int KT, uint16_t* lds, f32x16 (&acc)[TMI][TMJ],
-                                             float ident_v, int diag, int vwm, int vwn) {
+                                             int rows, int cols, float ident_v, int diag, int vwm, int vwn) {
   Pipe<RK, CK, IDENT, MASK, SHARED> p;
   p.rsrc_k = rsrc_k;
   p.rsrc_t = rsrc_t;
@@ -395,6 +404,14 @@ __device__ __forceinline__ void mainloop_run(const uint16_t* rsrc_k, const uint1
   p.KT = KT;
   p.lane = threadIdx.x & 63;
   p.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // its share of the direct loads
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int u = 2 * p.wave + q;
+    p.rk[q] = uint32_t(rows >= BM ? u : min(u, rows / 16 - 1)) * (16 * PANEL * 2);
+    p.ck[q] = uint32_t(cols >= BN ? u : min(u, cols / 16 - 1)) * (16 * PANEL * 2);
+  }
+  p.rt = uint32_t(rows >= BM ? p.wave : min(p.wave, rows / PANEL - 1)) * p.pstride_b;
+  p.ct = uint32_t(cols >= BN ? p.wave : min(p.wave, cols / PANEL - 1)) * p.pstride_b;
   p.wm = vwm;                                                 // its window of the output tile
   p.wn = vwn;
   p.lds = lds;
@@ -416,22 +433,32 @@ __device__ __forceinline__ void mainloop_run(const uint16_t* rsrc_k, const uint1
 // sym_diag (workgroup-uniform): a diagonal tile of a symmetric product, whose
 // work is dealt by diag_plan; SHARE: its row and column operands are the same
 // rows (SYRK, POLY: loaded once, Pipe SHARED), else two stacks' bands of the
-// same rows (SYMM).  idle (wave-uniform, full tiles only): the wave's window
-// holds only zero padding columns; it issues its share of the direct loads and
-// leaves its accumulators zero.
-template <int RK, int CK, int IDENT = IDENT_NONE, bool SHARE = true>
+// same rows (SYMM).  rows, cols: rows of the two operands that the stack holds
+// from the tile's first on (a multiple of 32; at most the tile's matter).  mv, nv:
+// those that are not padding; a wave whose window lies beyond them (as every window
+// whose identity columns lie beyond K does) issues its share of the direct loads and
+// leaves its accumulators zero (EDGE: there may be such windows).
+template <int RK, int CK, bool EDGE, int IDENT = IDENT_NONE, bool SHARE = true>
 __device__ __forceinline__ void mainloop(const uint16_t* rsrc_k, const uint16_t* rsrc_t, int thr_r,
                                          const uint16_t* csrc_k, const uint16_t* csrc_t, int thr_c,
                                          int64_t pstride, int KT, uint16_t* lds, f32x16 (&acc)[TMI][TMJ],
-                                         float ident_v = 0.f, int diag = 0, bool sym_diag = false,
-                                         bool idle = false) {
+                                         int rows, int cols, int mv, int nv, float ident_v = 0.f, int diag = 0,
+                                         bool sym_diag = false) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const WavePlan plan = sym_diag ? diag_plan(wave) : full_plan(wave);
+  const WavePlan plan = sym_diag ? diag_plan(wave) : full_plan(wave, mv);
+  const bool idle = EDGE && (plan.vwm * WM >= mv || plan.vwn * WN >= nv);
 #define MMUON_RUN(MASK, SH)                                                                                  \
-  mainloop_run<RK, CK, IDENT, MASK, SH>(rsrc_k, rsrc_t, thr_r, csrc_k, csrc_t, thr_c, pstride, KT, lds, acc, \
-                                        ident_v, diag, plan.vwm, plan.vwn)
-  if (!sym_diag && idle) MMUON_RUN(0, false);
-  else if (!sym_diag) MMUON_RUN(MASK_FULL, false);
+  mainloop_run<RK, CK, (MASK) != 0 ? IDENT : IDENT_NONE, MASK, SH>(rsrc_k, rsrc_t, thr_r, csrc_k, csrc_t, thr_c, \
+                                                                   pstride, KT, lds, acc, rows, cols, ident_v, diag, \
+                                                                   plan.vwm, plan.vwn)
+  if constexpr (EDGE) {
+    if (idle) {
+      if (sym_diag) MMUON_RUN(0, SHARE);
+      else MMUON_RUN(0, false);
+      return;
+    }
+  }
+  if (!sym_diag) MMUON_RUN(MASK_FULL, false);
   else if (plan.mask == MASK_FULL) MMUON_RUN(MASK_FULL, SHARE);
   else if (plan.mask == MASK_UPPER) MMUON_RUN(MASK_UPPER, SHARE);
   else if (plan.mask == MASK_LAST) MMUON_RUN(MASK_LAST, SHARE);
@@ -450,11 +477,11 @@ __device__ __forceinline__ void mainloop(const uint16_t* rsrc_k, const uint16_t*
 // both operands are one symmetric matrix, rounding-level apart for SYMM's two
 // commuting ones); its diagonal entries i = j < dlim get dadd added (in fp32,
 // before the rounding).
-__device__ __forceinline__ void stage_tile(char* stage, const f32x16 (&acc)[TMI][TMJ], float f,
+__device__ __forceinline__ void stage_tile(char* stage, const f32x16 (&acc)[TMI][TMJ], float f, int mv,
                                            bool diag = false, float dadd = 0.f, int dlim = 0) {
   const int tid = fresh_tid();
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const WavePlan plan = diag ? diag_plan(wave) : full_plan(wave);
+  const WavePlan plan = diag ? diag_plan(wave) : full_plan(wave, mv);
   const int wm = plan.vwm, wn = plan.vwn;
 #pragma unroll
   for (int i = 0; i < TMI; ++i) {
@@ -532,7 +559,7 @@ __device__ __forceinline__ void stage_tile(char* stage, const f32x16 (&acc)[TMI]
 // T[r][i] for the BN staged rows, dst at the first staged row of the tile's
 // first column panel (panel stride pstride).  One wave instruction writes rows
 // 16u .. 16u+15 of one panel (1 KiB contiguous).
-__device__ __forceinline__ void stage_rows(const char* stage, uint16_t* dst, int64_t pstride) {
+__device__ __forceinline__ void stage_rows(const char* stage, uint16_t* dst, int64_t pstride, int rows) {
   const int tid = fresh_tid();
   const int lane = tid & 63, wave = tid >> 6;
 #pragma unroll 4
@@ -540,6 +567,7 @@ __device__ __forceinline__ void stage_rows(const char* stage, uint16_t* dst, int
     const int u = wave + NWAVES * it;  // 8 panels x BN/16 row blocks
     const int q = u & 7, r = (u >> 3) * 16 + (lane >> 2);
     const int i = q * 32 + (lane & 3) * 8;
+    if (i >= rows || r >= rows) continue;  // beyond a partial tile
     const uint4 v = *reinterpret_cast<const uint4*>(stage + tile_off(r, i));
     *reinterpret_cast<uint4*>(dst + q * pstride + r * PANEL + (lane & 3) * 8) = v;
   }
@@ -583,9 +611,11 @@ __device__ __forceinline__ void stage_cols(const char* stage, Fn&& fn) {
 // from S1 and its column band from S2 in the same way.
 // ---------------------------------------------------------------------------
 static_assert(BM == BN, "square tiles: a symmetric tile is either diagonal or strictly upper");
-template <int STAGE>
+// PART: the stacks' extents are no multiples of the tile, so tiles at their ends are
+// partial; without it those checks are constants (they cost the 1024 x 1024 blocks 1%).
+template <int STAGE, bool PART>
 __device__ __forceinline__ void sym_work(const NsArgs& a, uint16_t* lds, int v) {
-  const int nt = a.mp / BM, nc = a.mp / BN;
+  const int nt = tiles_of(a.mp), nc = nt;
   const int tiles = nt * nc - R_SYM * nt * (nt - 1) / 2;
   int b, t;
   if (!decode_tile(v, tiles, a.N, b, t)) return;
@@ -608,18 +638,20 @@ __device__ __forceinline__ void sym_work(const NsArgs& a, uint16_t* lds, int v) 
   // on a diagonal tile only the 32 x 32 tiles on or above the diagonal are
   // computed; the others are staged from their transposes
   const bool diag = tc == ti;
+  const int rows = PART ? a.mp - r0 : BM, cols = PART ? a.mp - c0 : BN;
+  const int mv = PART ? a.m - r0 : BM, nv = PART ? a.m - c0 : BN;
   f32x16 acc[TMI][TMJ];
   if (STAGE == NS_SYRK)
-    mainloop<OP_K, OP_K>(src + r0 * PANEL, nullptr, 0, src + c0 * PANEL, nullptr, 0, pstride, K / BK, lds, acc,
-                         0.f, 0, diag);
+    mainloop<OP_K, OP_K, PART>(src + r0 * PANEL, nullptr, 0, src + c0 * PANEL, nullptr, 0, pstride, K / BK, lds, acc, rows,
+                         cols, mv, nv, 0.f, 0, diag);
   else if (STAGE == NS_POLY)  // acc = A A + (b/c) A, so P = c acc + a I = a I + b A + c A A
-    mainloop<OP_SPLIT, OP_SPLIT, IDENT_COL>(src + r0 * PANEL, src + (r0 / PANEL) * pstride, r0 / BK,
+    mainloop<OP_SPLIT, OP_SPLIT, PART, IDENT_COL>(src + r0 * PANEL, src + (r0 / PANEL) * pstride, r0 / BK,
                                             src + c0 * PANEL, src + (c0 / PANEL) * pstride, c0 / BK,
-                                            pstride, K / BK, lds, acc, a.cb / a.cc, c0, diag);
+                                            pstride, K / BK, lds, acc, rows, cols, mv, nv, a.cb / a.cc, c0, diag);
   else  // SYMM: acc = S1 S2; a diagonal tile loads both operands' bands
-    mainloop<OP_SPLIT, OP_SPLIT, IDENT_NONE, false>(src + r0 * PANEL, src + (r0 / PANEL) * pstride, r0 / BK,
+    mainloop<OP_SPLIT, OP_SPLIT, PART, IDENT_NONE, false>(src + r0 * PANEL, src + (r0 / PANEL) * pstride, r0 / BK,
                                                     src2 + c0 * PANEL, src2 + (c0 / PANEL) * pstride, c0 / BK,
-                                                    pstride, K / BK, lds, acc, 0.f, 0, diag);
+                                                    pstride, K / BK, lds, acc, rows, cols, mv, nv, 0.f, 0, diag);
 
   float f = STAGE == NS_POLY ? a.cc : 1.f;  // SYRK: s^2 on the first iteration
   if (STAGE == NS_SYRK && a.scale != nullptr) {
@@ -630,17 +662,17 @@ __device__ __forceinline__ void sym_work(const NsArgs& a, uint16_t* lds, int v) 
   char* stage = reinterpret_cast<char*>(lds);
   barrier();  // every wave is done with the ring
   // POLY: a on the diagonal of the m valid rows (the padding stays zero)
-  stage_tile(stage, acc, f, diag, STAGE == NS_POLY ? a.ca : 0.f, STAGE == NS_POLY ? a.m - r0 : 0);
+  stage_tile(stage, acc, f, mv, diag, STAGE == NS_POLY ? a.ca : 0.f, STAGE == NS_POLY ? a.m - r0 : 0);
   barrier_after_lds_writes();
   if (!diag) {
     // upper tile C[r0 + i][c0 + r] = T[r][i]
     uint16_t* dst = out + (c0 / PANEL) * pstride + int64_t(r0) * PANEL;
     stage_cols(stage, [&](int i, int r, const uint4& u) {
-      *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
+      if (i < rows && r < cols) *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
     });
   } else {
     // diagonal tile in full, through its mirror C[r0 + r][r0 + i] = T[r][i]
-    stage_rows(stage, out + (r0 / PANEL) * pstride + int64_t(r0) * PANEL, pstride);
+    stage_rows(stage, out + (r0 / PANEL) * pstride + int64_t(r0) * PANEL, pstride, rows);
   }
 }
 
@@ -648,8 +680,16 @@ template <int STAGE>
 __global__ __launch_bounds__(NT, WG_PER_CU) void ns_sym_bf16(NsArgs a, int total) {
   __shared__ __attribute__((aligned(1024))) uint16_t lds[LDS_ELEMS];
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
-    sym_work<STAGE>(a, lds, v);
+    sym_work<STAGE, false>(a, lds, v);
     barrier();  // the staging area is read before the next tile's loads refill the ring
+  }
+}
+template <int STAGE>
+__global__ __launch_bounds__(NT, WG_PER_CU) void ns_sym_edge_bf16(NsArgs a, int total) {
+  __shared__ __attribute__((aligned(1024))) uint16_t lds[LDS_ELEMS];
+  for (int v = blockIdx.x; v < total; v += gridDim.x) {
+    sym_work<STAGE, true>(a, lds, v);
+    barrier();
   }
 }
 
@@ -698,10 +738,10 @@ __device__ __forceinline__ void apply_chunk(typename TP::storage* prm, int64_t o
     if (e < valid) TP::store(prm, o + e, fmaf(alpha, u[e], TP::load(prm, o + e)));
 }
 
-template <int STAGE, bool TRANS, class TP>
+template <int STAGE, bool PART, bool TRANS, class TP>
 __device__ __forceinline__ void px_work(const NsArgs& a, uint16_t* lds, int v) {
-  const int tiles_i = a.mp / BM;
-  const int tiles = tiles_i * (a.np / BN);
+  const int tiles_i = tiles_of(a.mp);
+  const int tiles = tiles_i * tiles_of(a.np);
   int b, t;
   if (!decode_tile(v, tiles, a.N, b, t)) return;
   // column-band-major: the tiles_i tiles that read one column band of X are
@@ -718,11 +758,11 @@ __device__ __forceinline__ void px_work(const NsArgs& a, uint16_t* lds, int v) {
   const uint16_t* P = static_cast<const uint16_t*>(a.a_in) + int64_t(b) * a.mp * a.mp;
   const uint16_t* X = static_cast<const uint16_t*>(a.x_in) + int64_t(b) * a.mp * a.np + (c0 / PANEL) * pstride;
   f32x16 acc[TMI][TMJ];
-  // acc = P X; a wave whose 64 columns all lie in the zero padding (n <= column
-  // < np) computes nothing: its part of X' stays zero
-  const int wn = full_plan(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)).vwn;
-  mainloop<OP_SPLIT, OP_T>(P + r0 * PANEL, P + (r0 / PANEL) * pstride, r0 / BK, nullptr, X, 0, pstride, a.mp / BK,
-                           lds, acc, 0.f, 0, false, c0 + wn * WN >= a.n);
+  // acc = P X; a wave whose window lies in the zero padding computes nothing: its
+  // part of X' stays zero
+  const int rows = PART ? a.mp - r0 : BM, cols = PART ? a.np - c0 : BN, mv = PART ? a.m - r0 : BM;
+  mainloop<OP_SPLIT, OP_T, true>(P + r0 * PANEL, P + (r0 / PANEL) * pstride, r0 / BK, nullptr, X, 0, pstride, a.mp / BK,
+                           lds, acc, rows, cols, mv, a.n - c0);
 
   const float s = a.scale != nullptr ? a.scale[b] : 1.f;
   char* stage = reinterpret_cast<char*>(lds);
@@ -766,14 +806,14 @@ __device__ __forceinline__ void px_work(const NsArgs& a, uint16_t* lds, int v) {
     }
   }
   barrier();  // every wave is done with the ring
-  stage_tile(stage, acc, s);
+  stage_tile(stage, acc, s, mv);
   barrier_after_lds_writes();
   if (STAGE == NS_PX) {
     // X'[r0 + i][c0 + r] = T[r][i]
     uint16_t* dst = static_cast<uint16_t*>(a.out) + int64_t(b) * a.mp * a.np + (c0 / PANEL) * pstride +
                     int64_t(r0) * PANEL;
     stage_cols(stage, [&](int i, int r, const uint4& u) {
-      *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
+      if (i < rows && r < cols) *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
     });
     return;
   }
@@ -840,8 +880,16 @@ template <int STAGE, bool TRANS, class TP>
 __global__ __launch_bounds__(NT, WG_PER_CU) void ns_px_bf16(NsArgs a, int total) {
   __shared__ __attribute__((aligned(1024))) uint16_t lds[LDS_ELEMS];
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
-    px_work<STAGE, TRANS, TP>(a, lds, v);
+    px_work<STAGE, false, TRANS, TP>(a, lds, v);
     barrier();  // the staging area is read before the next tile's loads refill the ring
+  }
+}
+template <int STAGE, bool TRANS, class TP>
+__global__ __launch_bounds__(NT, WG_PER_CU) void ns_px_edge_bf16(NsArgs a, int total) {
+  __shared__ __attribute__((aligned(1024))) uint16_t lds[LDS_ELEMS];
+  for (int v = blockIdx.x; v < total; v += gridDim.x) {
+    px_work<STAGE, true, TRANS, TP>(a, lds, v);
+    barrier();
   }
 }
 
@@ -1345,21 +1393,26 @@ __global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(2))) void 
   }
 }
 
+// The kernels with partial tiles where the stacks' extents ask for them.
 template <int STAGE, class TP>
 void launch_bf16(const NsArgs& a, hipStream_t s) {
   const int nb8 = 8 * ((a.N + 7) / 8);
+  const bool edge_m = a.mp % BM != 0;
   if constexpr (STAGE == NS_SYRK || STAGE == NS_POLY || STAGE == NS_SYMM) {
-    const int nt = a.mp / BM;
-    const int nc = a.mp / BN;
+    const int nt = tiles_of(a.mp), nc = nt;
     const int total = nb8 * (nt * nc - R_SYM * nt * (nt - 1) / 2);
-    hipLaunchKernelGGL((ns_sym_bf16<STAGE>), dim3(resident_grid(total)), dim3(NT), 0, s, a, total);
-  } else {
-    const int total = nb8 * (a.mp / BM) * (a.np / BN);
     const dim3 grid(resident_grid(total));
-    if constexpr (STAGE == NS_PX) {
-      hipLaunchKernelGGL((ns_px_bf16<STAGE, false, TP>), grid, dim3(NT), 0, s, a, total);
-    } else {
-      if (!a.transposed) hipLaunchKernelGGL((ns_px_bf16<STAGE, false, TP>), grid, dim3(NT), 0, s, a, total);
+    if (edge_m) hipLaunchKernelGGL((ns_sym_edge_bf16<STAGE>), grid, dim3(NT), 0, s, a, total);
+    else hipLaunchKernelGGL((ns_sym_bf16<STAGE>), grid, dim3(NT), 0, s, a, total);
+  } else {
+    const int total = nb8 * tiles_of(a.mp) * tiles_of(a.np);
+    const dim3 grid(resident_grid(total));
+    const bool edge = edge_m || a.np % BN != 0;
+    if (STAGE == NS_PX || !a.transposed) {
+      if (edge) hipLaunchKernelGGL((ns_px_edge_bf16<STAGE, false, TP>), grid, dim3(NT), 0, s, a, total);
+      else hipLaunchKernelGGL((ns_px_bf16<STAGE, false, TP>), grid, dim3(NT), 0, s, a, total);
+    } else if constexpr (STAGE == NS_PX_APPLY) {
+      if (edge) hipLaunchKernelGGL((ns_px_edge_bf16<STAGE, true, TP>), grid, dim3(NT), 0, s, a, total);
       else hipLaunchKernelGGL((ns_px_bf16<STAGE, true, TP>), grid, dim3(NT), 0, s, a, total);
     }
   }
@@ -1397,8 +1450,11 @@ void launch_f32(const NsArgs& a, hipStream_t s) {
 
 }  // namespace
 
-int ns_tile_m(int ns_dtype) { return ns_dtype == MMUON_BF16 ? BM : F_PAD; }
-int ns_tile_n(int ns_dtype) { return ns_dtype == MMUON_BF16 ? 256 : F_PAD; }  // pack tiles 256 columns
+// bf16: 64, two K slices, so that the stacks' traffic, the K extents and the waves'
+// work follow the block's sides (264 blocks of 384 x 384 padded to 384 instead of 512:
+// PX 88 -> 60 us, 4.9 TB/s; SYRK 57 -> 48, POLY 70 -> 50, pack 120 -> 95); beyond 2048
+// whole tiles, which the kernels without partial ones take (at most an eighth of padding).
+int ns_pad(int ns_dtype, int side) { return ns_dtype != MMUON_BF16 ? F_PAD : side <= 2048 ? 64 : 256; }
 int ns_tile_k(int ns_dtype) { return ns_dtype == MMUON_BF16 ? BK : FK; }
 
 int launch_ns_stage(const NsArgs& a, int stage, int ns_dtype, int param_dtype, hipStream_t s) {

@@ -137,6 +137,72 @@ def test_stage_outputs_against_fp64_products(shape):
         assert float(pa[:, lay.m:, :].abs().max()) == 0.0 and float(ap[:, :, lay.m:].abs().max()) == 0.0
 
 
+# sides whose last 256-wide tile holds 64, 128, 192 or 256 rows or columns, K extents from two slices on
+@pytest.mark.parametrize("shape", [(2, 8, 16), (3, 64, 64), (2, 72, 200), (2, 200, 72), (2, 264, 264), (2, 328, 520),
+                                   (3, 384, 384), (2, 384, 1024), (2, 1000, 344), (2, 456, 1368), (2, 520, 2056),
+                                   (2, 760, 984), (70, 384, 384)], ids=lambda s: "x".join(map(str, s)))
+def test_partial_tiles_against_fp64_products(shape):
+    """SYRK, POLY, PX (and SYMM where its stacks fit) of blocks whose padded sides are no multiple of the tile, as in
+    the test above: every stored entry against the fp64 product of the stage's own inputs, zero padding, exactly
+    symmetric diagonal tiles; whatever the stacks held before (here NaN) does not enter."""
+    gen = torch.Generator().manual_seed(9)
+    g = (torch.randn(shape, generator=gen) * 1e-3).to(DEV)
+    p = torch.zeros_like(g, dtype=torch.bfloat16)
+    grad, buf = g.bfloat16(), torch.zeros_like(g)
+    (gl,) = MuonPlanner().plan([p], [grad], [buf], torch.bfloat16)
+    lib, stream = _abi.lib(), _abi.stream_handle(DEV)
+    coeffs = (C.c_float * 3)(*NS_COEFFS)
+    a_c, b_c, c_c = NS_COEFFS
+    lay, ws, nb = gl.ws.layout, gl.ws, gl.nblocks
+    mp, np_ = lay.mp, lay.np_
+    assert mp >= lay.m and np_ >= lay.n and mp % 64 == 0 and np_ % 64 == 0
+    for t in (ws.x0, ws.x1, ws.a, ws.p):
+        t.view(torch.bfloat16).fill_(float("nan"))
+
+    def run(kind, in0, in1, out, scaled=0):
+        op = _abi.NsOp(kind, in0, in1, out, scaled, 0)
+        _abi.check(lib.mmuon_ns_run_op(C.byref(gl.struct), C.byref(op), coeffs, C.c_float(0.0), stream), "run_op")
+        torch.cuda.synchronize()
+
+    tile = torch.arange(mp, device=DEV) // TILE
+    stored = tile[:, None] <= tile[None, :]
+
+    def check(got, ref, what):
+        for b in range(nb):
+            err = (got[b] - ref[b]).abs().masked_fill(~stored, 0.0).max()
+            assert err <= 2.0 ** -8 * ref[b].abs().max(), f"{what} block {b}: {err:.3e}"
+        same = tile[:, None] == tile[None, :]
+        assert torch.equal(got.masked_fill(~same, 0.0), got.transpose(1, 2).masked_fill(~same, 0.0)), what
+
+    def full(a):
+        return torch.where(stored, a, a.transpose(1, 2))
+
+    _abi.check(lib.mmuon_momentum_pack(C.byref(gl.struct), 0.0, stream), "pack")
+    torch.cuda.synchronize()
+    s = ws.scale.double().view(nb, 1, 1)
+    x = panels(ws.x0, nb, mp, np_)
+    gx = grad.double()
+    gx = gx.transpose(1, 2) if gl.transposed else gx
+    assert torch.equal(x[:, :lay.m, :lay.n], gx) and not x[:, lay.m:].any() and not x[:, :, lay.n:].any()
+    run(_abi.NSOP_SYRK, _abi.NSB_X0, -1, _abi.NSB_A, 1)
+    a = full(panels(ws.a, nb, mp, mp))
+    check(a, s * s * (x @ x.transpose(1, 2)), "SYRK")
+    run(_abi.NSOP_POLY, _abi.NSB_A, -1, _abi.NSB_P)
+    pm = full(panels(ws.p, nb, mp, mp))
+    eye = torch.diag((torch.arange(mp, device=DEV) < lay.m).double())
+    check(pm, a_c * eye + b_c * a + c_c * (a @ a), "POLY")
+    assert not pm[:, lay.m:].any() and not pm[:, :, lay.m:].any()
+    run(_abi.NSOP_PX, _abi.NSB_P, _abi.NSB_X0, _abi.NSB_X1, 1)
+    ref, got = s * (pm @ x), panels(ws.x1, nb, mp, np_)
+    for b in range(nb):
+        assert (got[b] - ref[b]).abs().max() <= 2.0 ** -8 * ref[b].abs().max(), f"PX block {b}"
+    assert not got[:, lay.m:].any() and not got[:, :, lay.n:].any()
+    if np_ >= 2 * mp:
+        run(_abi.NSOP_SYMM, _abi.NSB_P, _abi.NSB_A, _abi.NSB_X1_S1)
+        sub = ws.x1.view(torch.bfloat16)[nb * mp * mp: 2 * nb * mp * mp]
+        check(full(panels(sub, nb, mp, mp)), pm @ a, "SYMM")
+
+
 def test_run_op_rejects_invalid_ops():
     """mmuon_ns_run_op validates buffer kinds, overlaps and sub-stack room on the
     host before any launch."""
