@@ -108,17 +108,33 @@ __device__ __forceinline__ int64_t mn_off(const GOp& o, int64_t m) {
   const int64_t s = seg_div(m, o.mmagic);
   return s * o.mseg_stride + (m - s * o.mseg) * o.mstride;
 }
-// The K addressing of an operand, held by the main loop.
-struct GOpK {
-  int64_t kstride, kseg_stride;
-  uint64_t kmagic;
-  int64_t kseg;
+// An operand's walk over K, one slice of BK at a time.  Segments are whole slices
+// (multiples of 32), so a slice lies in one.  (Forming each slice's address from its
+// index, a 64-bit division and three products, and testing every load for the end of K
+// paced the small tiles: 8 tokens of 4 x 1024 x 1024 11.5 -> 10.4 us, 500 tokens of 4 x
+// 512 x 1376 12.7 -> 11.4.  Rings of 8 or 16 slots, and reading a whole slice's fragments
+// behind the barrier, did not help them.)
+struct KWalk {
+  const char* p;       // the slice's first element (tile row 0)
+  int64_t step, wrap;  // bytes to the next slice, and beyond that into the next segment
+  int pos, seg;        // the slice's place in its segment, the segment's length
+  __device__ __forceinline__ void start(const GOp& o, const char* base, int k) {
+    const int64_t s = seg_div(k, o.kmagic);
+    pos = k - int(s) * o.kseg;
+    seg = o.kseg;
+    p = base + s * o.kseg_stride + int64_t(pos) * o.kstride;
+    step = int64_t(BK) * o.kstride;
+    wrap = o.kseg_stride - int64_t(o.kseg) * o.kstride;
+  }
+  __device__ __forceinline__ void next() {
+    p += step;
+    pos += BK;
+    if (pos == seg) {
+      p += wrap;
+      pos = 0;
+    }
+  }
 };
-__device__ __forceinline__ GOpK k_addr(const GOp& o) { return GOpK{o.kstride, o.kseg_stride, o.kmagic, o.kseg}; }
-__device__ __forceinline__ int64_t k_off(const GOpK& o, int64_t k) {
-  const int64_t s = seg_div(k, o.kmagic);
-  return s * o.kseg_stride + (k - s * o.kseg) * o.kstride;
-}
 
 // bf16 result: row m of batch g at base + g bstride + seg(m), column n at
 // 2 n; riffle (log2 l > 0): column jq of the tile's columns goes to plane
@@ -186,11 +202,11 @@ struct GPipe {
     bf16x8 c[WJ];
   };
   typedef f32x16 Acc[WI][WJ];
-  const char* abase;  // row operand at (tile row 0, k = 0) of this batch
-  const char* bbase;
-  GOpK ak, bk;        // K addressing of the two operands
+  KWalk ak, bk;            // the slice to load next, of the two operands
+  int nxt;                 // its index (the last slice stays: it refills consumed slots)
   uint32_t loff[GE::DMA];  // per-lane byte offsets of the loads (OOB: beyond the extent)
-  int kbeg, kend, KT;
+  uint32_t tail[GE::DMA];  // OOB where the load's element lies beyond the last slice's K
+  int KT;
   int wave, lane, wm, wn;
   char* lds;
   uint32_t lds0;
@@ -201,33 +217,31 @@ struct GPipe {
     return reinterpret_cast<const uint16_t*>(lds + (uint32_t(kt) % RING) * GE::SLOTB);
   }
 
-  // Load Q (row operand first) of slice src_kt into the slot of slice slot_kt.
+  // Load Q (row operand first) of the next slice into the slot of slice slot_kt.
   // Load u = RL wave + Q (CL wave + Q - RL) of the operand's BM / 16 (BN / 16).
   // K form: operand rows 16 u + lane/4, chunk (lane%4) ^ ((lane>>4)&3); T form: k rows
   // 16 (u%2) + lane/4 of the slice, MN 32 (u/2) + 8 (lane%4).  Either way the load
   // lands at byte 1024 u of the operand's slice.
   template <int Q>
-  __device__ __forceinline__ void issue_one(int src_kt, int slot_kt) const {
+  __device__ __forceinline__ void issue_one(int slot_kt) const {
     constexpr bool ROW = Q < GE::RL;
-    constexpr bool T = ROW ? AT : BT;
     const int u = ROW ? GE::RL * wave + Q : GE::CL * wave + Q - GE::RL;
     const uint32_t dst = lds0 + (uint32_t(slot_kt) % RING) * GE::SLOTB + (ROW ? 0 : GE::RSLB) + u * 1024;
-    const int k0 = kbeg + src_kt * BK;
-    const char* sb = (ROW ? abase : bbase) + k_off(ROW ? ak : bk, k0);
-    uint32_t voff = loff[Q];
-    const int rem = kend - k0;
-    if (rem < BK) {
-      // K delta of this lane's load within the slice: K form, its 8-element chunk; T form, its k row
-      const int kd = T ? 16 * (u & 1) + (lane >> 2) : 8 * ((lane & 3) ^ ((lane >> 4) & 3));
-      if (kd >= rem) voff = OOB;
-    }
-    bdma16(buffer_rsrc(sb), voff, dst);
+    const uint32_t last = nxt == KT - 1 ? OOB : 0;
+    bdma16(buffer_rsrc(ROW ? ak.p : bk.p), loff[Q] | (tail[Q] & last), dst);
   }
   template <int Q0, int Q1>
-  __device__ __forceinline__ void issue(int src_kt, int slot_kt) const {
+  __device__ __forceinline__ void issue(int slot_kt) const {
     if constexpr (Q0 < Q1) {
-      issue_one<Q0>(src_kt, slot_kt);
-      issue<Q0 + 1, Q1>(src_kt, slot_kt);
+      issue_one<Q0>(slot_kt);
+      issue<Q0 + 1, Q1>(slot_kt);
+    }
+  }
+  __device__ __forceinline__ void advance() {
+    if (nxt + 1 < KT) {
+      ak.next();
+      bk.next();
+      ++nxt;
     }
   }
 
@@ -252,40 +266,43 @@ struct GPipe {
   // MFMA g of a k step, with its share of the fragment reads of the next step and,
   // in the second k step, of the direct loads
   template <int KK, int g>
-  __device__ __forceinline__ void half(int kt, int src, int slt, const Fr& f, Fr& n, Acc& acc) const {
+  __device__ __forceinline__ void half(int kt, const Fr& f, Fr& n, Acc& acc) const {
     if constexpr (g < NM) {
       acc[g / WJ][g % WJ] = mfma(f.r[g / WJ], f.c[g % WJ], acc[g / WJ][g % WJ]);
       if constexpr (KK == 0) {
         load<1, g * NR / NM, (g + 1) * NR / NM>(kt, n);
       } else {
         load<0, g * NR / NM, (g + 1) * NR / NM>(kt + 1, n);
-        issue<g * GE::DMA / NM, (g + 1) * GE::DMA / NM>(src, slt);
+        issue<g * GE::DMA / NM, (g + 1) * GE::DMA / NM>(kt + RING - 1);
       }
       __builtin_amdgcn_sched_barrier(0);
-      half<KK, g + 1>(kt, src, slt, f, n, acc);
+      half<KK, g + 1>(kt, f, n, acc);
     }
   }
 
-  __device__ __forceinline__ void body(int kt, Fr& fa, Fr& fb, Acc& acc) const {
-    half<0, 0>(kt, 0, 0, fa, fb, acc);
+  __device__ __forceinline__ void body(int kt, Fr& fa, Fr& fb, Acc& acc) {
+    half<0, 0>(kt, fa, fb, acc);
     wait_vm<(RING - 3) * GE::DMA>();  // slice kt+1 landed
     barrier();
-    const int src = kt + RING - 1 < KT ? kt + RING - 1 : KT - 1;
     // raised wave priority from the barrier to the end of k step 1, so the
     // SIMD's wave still in this phase wins issue over one already in the next
     // step and catches up before the next barrier
     __builtin_amdgcn_s_setprio(1);
-    half<1, 0>(kt, src, kt + RING - 1, fb, fa, acc);
+    half<1, 0>(kt, fb, fa, acc);
     __builtin_amdgcn_s_setprio(0);
+    advance();
   }
 
-  __device__ __forceinline__ void run(Acc& acc) const {
+  __device__ __forceinline__ void run(Acc& acc) {
 #pragma unroll
     for (int i = 0; i < WI; ++i)
 #pragma unroll
       for (int j = 0; j < WJ; ++j) acc[i][j] = f32x16{};
 #pragma unroll
-    for (int q = 0; q < RING - 1; ++q) issue<0, GE::DMA>(q < KT ? q : KT - 1, q);
+    for (int q = 0; q < RING - 1; ++q) {
+      issue<0, GE::DMA>(q);
+      advance();
+    }
     wait_vm<(RING - 2) * GE::DMA>();  // slice 0 landed
     barrier();
     Fr fa, fb;
@@ -413,17 +430,21 @@ __device__ __forceinline__ void gemm_work(const GemmArgs& a, char* lds, int v) {
   p.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   p.wm = p.wave / GE::GN;
   p.wn = p.wave % GE::GN;
-  p.ak = k_addr(a.a);
-  p.bk = k_addr(a.b);
-  p.abase = a.a.base + int64_t(g) * a.a.bstride + mn_off(a.a, m0);
-  p.bbase = a.b.base + int64_t(g) * a.b.bstride + mn_off(a.b, n0);
-  p.kbeg = sp * a.kchunk;
-  p.kend = min(a.K, p.kbeg + a.kchunk);
-  p.KT = (p.kend - p.kbeg + BK - 1) / BK;
+  const int kbeg = sp * a.kchunk, kend = min(a.K, kbeg + a.kchunk);
+  p.ak.start(a.a, a.a.base + int64_t(g) * a.a.bstride + mn_off(a.a, m0), kbeg);
+  p.bk.start(a.b, a.b.base + int64_t(g) * a.b.bstride + mn_off(a.b, n0), kbeg);
+  p.nxt = 0;
+  p.KT = (kend - kbeg + BK - 1) / BK;
+  const int rem = kend - kbeg - (p.KT - 1) * BK;  // K of the last slice
 #pragma unroll
-  for (int q = 0; q < GE::RL; ++q) p.loff[q] = lane_offset<AT>(a.a, m0, GE::RL * p.wave + q, p.lane);
-#pragma unroll
-  for (int q = 0; q < GE::CL; ++q) p.loff[GE::RL + q] = lane_offset<BT>(a.b, n0, GE::CL * p.wave + q, p.lane);
+  for (int q = 0; q < GE::DMA; ++q) {
+    const bool row = q < GE::RL;
+    const int u = row ? GE::RL * p.wave + q : GE::CL * p.wave + q - GE::RL;
+    p.loff[q] = row ? lane_offset<AT>(a.a, m0, u, p.lane) : lane_offset<BT>(a.b, n0, u, p.lane);
+    // K delta of this lane's load within a slice: K form, its 8-element chunk; T form, its k row
+    const int kd = (row ? AT : BT) ? 16 * (u & 1) + (p.lane >> 2) : 8 * ((p.lane & 3) ^ ((p.lane >> 4) & 3));
+    p.tail[q] = kd >= rem ? OOB : 0;
+  }
   p.lds = lds;
   p.lds0 = lds_addr(lds);
 #pragma unroll
