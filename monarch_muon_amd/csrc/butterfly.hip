@@ -19,7 +19,8 @@
 // back in place.  bf16 operands, fp32 accumulation, bf16 results (the rounding
 // points of the reference's bf16 bmms: out1, out, dt, dx, dw1, dw2).
 //
-// One GEMM kernel serves all six products, in 256-, 128- and 64-wide tiles (gemm_plan
+// One GEMM kernel serves the six products (a second one the forward's two for a few
+// tokens), in 256-, 128- and 64-wide tiles (gemm_plan
 // picks by the shapes): the MFMA pipeline and LDS slice forms of mfma_tile.hpp,
 // operands K-major (K form) or MN-major (T form, read transposed with
 // ds_read_b64_tr_b16), staged by buffer loads straight into LDS.  A buffer load
@@ -32,12 +33,13 @@
 // backward splits dout's blocks in one pass (to_blocks_kernel).
 //
 // What bounds it, one 6.89B up-projection (4 x 1024 x 1024, 4 x 2752 x 1024) at 4096
-// tokens, forward + backward 563 -> 465 us with the output stored in feature order
+// tokens, forward + backward 563 -> 453 us with the output stored in feature order
 // (two strided copies of 63-72 us before, one pass of 27-35 now): the 256-wide products
 // spend 8 us of a 45 us round filling and draining the pipeline, and read and write LDS
 // as long as their MFMAs run.  At 4096 tokens of 4 x 512 x 512 the 128-wide tiles took
 // the six products from 157 to 121 us, at 1000 tokens of 2 x 256 x 256 the 64-wide ones
-// from 125 to 52, at 8 tokens of the 6.89B layer (two products) from 53 to 22.
+// from 125 to 52.  Up to 64 tokens the forward's two products have a kernel of their
+// own (butterfly_few).
 #include <algorithm>
 #include <atomic>
 
@@ -524,6 +526,101 @@ __global__ __launch_bounds__(GE::NTH, GE::PER_CU * GE::NW / 4) void butterfly_ge
   }
 }
 
+// ---------------------------------------------------------------------------
+// The forward products for a few tokens (generation): 16 features x 16 NT tokens per
+// workgroup, whose waves split K and add their fp32 partials in wave order.
+//
+// Bound by the weights' read.  A 64-wide tile leaves most of the chip idle here (4 x
+// 1024 features are 64 workgroups) and walks all of K behind a barrier per slice; with
+// 16 features per workgroup and an eighth of K per wave, every wave streams its own
+// slices through its own ring, without barriers, and 256 workgroups have 24 KiB and
+// more in flight each.  Forward of the 6.89B up-projection at 1 / 8 / 32 / 64 tokens 26 / 26
+// / 26 / 27 -> 12 / 13 / 16 / 22 us, the 1.3B query 13.5 / 13.7 / 14 / 14 -> 6.6 / 7.0 /
+// 8.2 / 10.5, the toy up-projection 9.5 / 9.8 / 10.2 / 10.3 -> 6.0 / 6.2 / 6.6 / 7.9.
+// The slices go through LDS because fragment loads straight into registers put
+// neighbouring lanes in different rows: 64 tokens of the first 27 us.  Short rings: more
+// workgroups per CU are worth more than deeper ones (64 tokens: 25 us with 4 slots).
+// Each workgroup reads all tokens again, which is what grows with them; from 128 on
+// the tiles are as fast (28 us).
+// ---------------------------------------------------------------------------
+constexpr int FEW_W = 8;        // waves of a workgroup, which share K
+constexpr int FEW_TOKENS = 64;  // largest number of tokens
+constexpr int FEW_K = 32;       // k of a step
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int NT, bool FEATURES>
+__global__ __launch_bounds__(64 * FEW_W) void butterfly_few(GemmArgs a) {
+  constexpr int RING = NT == 1 ? 3 : 2, DMA = 1 + NT;  // K steps in flight per wave, 1 KiB loads of a step
+  constexpr int LD = 20;  // floats per token of a staged partial (16 features; rows start on different banks)
+  constexpr int WLDS = RING * DMA * 1024, RED = FEW_W * NT * 16 * LD * 4;
+  __shared__ __attribute__((aligned(1024))) char lds[FEW_W * WLDS > RED ? FEW_W * WLDS : RED];
+  const int g = blockIdx.x / a.tiles_n, n0 = (blockIdx.x % a.tiles_n) * 16;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const i32x4 wr = buffer_rsrc(a.b.base + int64_t(g) * a.b.bstride + n0 * a.b.mstride);
+  const i32x4 xr = buffer_rsrc(a.a.base + int64_t(g) * a.a.bstride);
+  // loads: row lane/4, 16-B chunk of the step's 64 B at (lane%4) ^ (row/4)%4
+  const int lrow = lane >> 2, lk = ((lane & 3) ^ ((lane >> 4) & 3)) * 8;
+  uint32_t ro[DMA];
+  ro[0] = n0 + lrow < a.N ? uint32_t(lrow * a.b.mstride) : OOB;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) ro[1 + t] = t * 16 + lrow < a.M ? uint32_t((t * 16 + lrow) * a.a.mstride) : OOB;
+  const int kbeg = wave * a.kchunk, kend = min(a.K, kbeg + a.kchunk);
+  char* const ring = lds + wave * WLDS;
+  const uint32_t ring0 = lds_addr(ring);
+  auto issue = [&](int k, int slot) {
+    const uint32_t ko = k + lk < kend ? uint32_t(k + lk) * 2 : OOB;
+#pragma unroll
+    for (int q = 0; q < DMA; ++q)
+      bdma16(q == 0 ? wr : xr, (ro[q] | ko) & OOB ? OOB : ro[q] + ko, ring0 + (slot * DMA + q) * 1024);
+  };
+  // fragments: row lane%16, k 8 (lane/16) .. +7
+  const int l16 = lane & 15;
+  const uint32_t frag = uint32_t(l16 * 64 + (((lane >> 4) ^ (l16 >> 2)) << 4));
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{};
+  if (kbeg < kend) {
+#pragma unroll
+    for (int q = 0; q < RING; ++q) issue(kbeg + FEW_K * q, q);
+    int slot = 0;
+    for (int k = kbeg; k < kend; k += FEW_K) {
+      wait_vm<(RING - 1) * DMA>();
+      const char* s = ring + slot * DMA * 1024 + frag;
+      const bf16x8 w = *reinterpret_cast<const bf16x8*>(s);
+      bf16x8 x[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) x[t] = *reinterpret_cast<const bf16x8*>(s + (1 + t) * 1024);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the slot is loaded again
+      issue(k + FEW_K * RING, slot);
+      slot = slot + 1 == RING ? 0 : slot + 1;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[t], acc[t], 0, 0, 0);
+    }
+    wait_vm<0>();
+  }
+  __syncthreads();
+  // lane: token l16, features 4 (lane/16) .. +3
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    *reinterpret_cast<f32x4*>(red + ((wave * NT + t) * 16 + l16) * LD + (lane >> 4) * 4) = acc[t];
+  __syncthreads();
+  for (int i = threadIdx.x; i < NT * 256; i += 64 * FEW_W) {
+    const int f = i & 15, tok = i >> 4, col = n0 + f;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < FEW_W; ++w) v += red[(w * NT * 16 + tok) * LD + f];
+    if (tok >= a.M || col >= a.N) continue;
+    char* dst = a.c.base + int64_t(tok) * a.c.rstride;
+    if (FEATURES)
+      dst += (int64_t(col) * a.G + g) * 2;
+    else
+      dst += int64_t(g) * a.c.bstride + (col & ((1 << a.c.log2l) - 1)) * a.c.cplane + int64_t(col >> a.c.log2l) * 2;
+    *reinterpret_cast<uint16_t*>(dst) = f2bf(v);
+  }
+}
+
 // Split-K reduction: out row seg(m) of batch g, columns n..n+7 =
 // bf16(sum over splits, in split order, of the fp32 partials).  S = 0 writes zeros.
 __global__ __launch_bounds__(256) void splitk_reduce(const float* partial, int S, int G, int M, int N, GOut c) {
@@ -701,6 +798,16 @@ void launch_gemm_t(const GemmArgs& a, hipStream_t s) {
   else launch_gemm_g<G64, AT, BT, OUT>(a, s);
 }
 
+template <bool FEATURES>
+void launch_few(GemmArgs a, hipStream_t s) {
+  a.tiles_n = cdiv(a.N, 16);
+  a.kchunk = cdiv(a.K, FEW_K * FEW_W) * FEW_K;
+  const dim3 grid(unsigned(a.G * a.tiles_n)), block(64 * FEW_W);
+  if (a.M <= 16) hipLaunchKernelGGL((butterfly_few<1, FEATURES>), grid, block, 0, s, a);
+  else if (a.M <= 32) hipLaunchKernelGGL((butterfly_few<2, FEATURES>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((butterfly_few<4, FEATURES>), grid, block, 0, s, a);
+}
+
 void launch_reduce(const GemmArgs& a, const GOut& c, hipStream_t s) {
   const int64_t total = int64_t(a.G) * a.M * (a.N / 8);
   const int blocks = int(std::min<int64_t>(std::max<int64_t>(1, (total + 255) / 256), 8192));
@@ -761,13 +868,17 @@ int launch_butterfly_fwd(const mmuon_butterfly_args& x, bool features, hipStream
   f1.c = make_out(x.out1, ql * 2, int64_t(d.q) * 2, UNSEG, 0, d.log2l, d.B * d.q * 2);
   // (a 64-wide tile of 16 planes would write runs shorter than 16 B)
   set_geometry(f1, int(d.B), d.q, d.p, d.nb, gemm_plan(d.B, d.q, d.nb, d.p, false, d.nb > 8));
-  launch_gemm_t<false, false, OUT_TILE>(f1, st);
+  const bool few = d.B <= FEW_TOKENS;
+  if (few) launch_few<false>(f1, st);
+  else launch_gemm_t<false, false, OUT_TILE>(f1, st);
   GemmArgs f2{};  // out[:, ll] = t[ll] . w2[ll]^T
   f2.a = make_op(x.out1, d.B * d.q * 2, int64_t(d.q) * 2, 2, int(d.B));
   f2.b = make_op(x.w2, int64_t(d.s) * d.q * 2, int64_t(d.q) * 2, 2, d.s);
   f2.c = make_out(x.out, int64_t(d.s) * 2, int64_t(d.nb) * d.s * 2);
   set_geometry(f2, int(d.B), d.s, d.q, d.nb, gemm_plan(d.B, d.s, d.nb, d.q, false));
-  if (features && d.nb > 1) launch_gemm_t<false, false, OUT_FEATURES>(f2, st);
+  if (few && features && d.nb > 1) launch_few<true>(f2, st);
+  else if (few) launch_few<false>(f2, st);
+  else if (features && d.nb > 1) launch_gemm_t<false, false, OUT_FEATURES>(f2, st);
   else launch_gemm_t<false, false, OUT_TILE>(f2, st);
   return 0;
 }

@@ -106,6 +106,32 @@ def test_layer_form_equals_the_blocked_pair(case):
             assert rel(u, v) <= TOL
 
 
+@pytest.mark.parametrize("tokens", [1, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("dims", [(2, 64, 136, 72), (4, 256, 344, 1096), (1, 1024, 1024, 520), (16, 512, 264, 56)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_forward_for_few_tokens(tokens, dims):
+    """The few-token kernel at the edges of its token tiles, with fewer and more K steps than its waves' rings hold,
+    features and K that end inside a tile, and inputs that fill no tile: rows beyond the tokens must not be read into
+    the result (the poison behind them is NaN).  fp32 products of bf16 inputs, rounded once: each result within half
+    a bf16 step of the exact sum, a step at a rounding boundary (2^-8 of it), and fp32 summation noise."""
+    print("few tokens", tokens, dims, flush=True)
+    nb, q, p, s = dims
+    x, w1, w2, _ = make(tokens, nb, q, p, s, seed=tokens)
+    hold = torch.full((80, nb * p), float("nan"), dtype=torch.bfloat16, device=DEV)
+    hold[:tokens] = x.to(DEV)
+    w1g, w2g = gpu(w1, w2)
+    out, out1 = butterfly_blk_op(hold[:tokens], w1g, w2g)
+    y = butterfly_blk(hold[:tokens], w1g, w2g)
+    torch.cuda.synchronize()
+    mid = torch.einsum("bkp,kqp->bkq", x.double().view(tokens, nb, p), w1.double())  # out1[b][kk][jq]
+    t = mid.reshape(tokens, q, nb).permute(2, 0, 1)                                  # the riffle: t[ll][b][i]
+    got1 = out1.cpu().double()
+    assert torch.all((got1.reshape(t.shape) - t).abs() <= t.abs() * 2.0 ** -8 + p * 2.0 ** -22)
+    ref = torch.einsum("lbi,lsi->bls", got1.reshape(t.shape), w2.double())
+    assert torch.all((out.cpu().double().reshape(ref.shape) - ref).abs() <= ref.abs() * 2.0 ** -8 + q * 2.0 ** -22)
+    assert torch.equal(y, out.transpose(1, 2).reshape(tokens, s * nb))
+
+
 @pytest.mark.parametrize("how", ["compile", "saved_hooks", "expanded_grad", "second_order"])
 def test_layer_operator_under_torch(how):
     """The native operator traced by torch.compile, with saved-tensor hooks and with a gradient that is no dense
