@@ -44,7 +44,7 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "optimizer-step ms, 6.89B-ref nb=4 bf16; NS TFLOP/s as % of bf16 MFMA peak"
 PEAK_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
-PEAK_F32_TFLOPS = 157.3     # MI355X dense fp32 MFMA
+PEAK_F32_TFLOPS = PEAK_BF16_TFLOPS / 6  # an fp32 product is six bf16 MFMA products (the fp32 MFMA: 157.3)
 PEAK_HBM_GBS = 8000.0
 REFERENCE_H100_MS = 304.4   # README.md:16 (bf16 momentum, H100)
 
@@ -149,7 +149,11 @@ def kernel_symbol(kind, gl, it, fp8=False):
     tp = "BF16T" if gl is not None and gl.struct.param_dtype == 1 else "F32T"
     if gl is not None and kind in NS_KINDS and gl.struct.ns_dtype == 0:  # fp32 Newton-Schulz
         stage = {"syrk": 0, "poly": 1, "px": 2, "px_apply": 3}[kind]
-        return f"ns_f32<{stage}, {tp if stage == 3 else 'F32T'}>"
+        lay, sym = gl.ws.layout, stage < 2
+        nt = lay.mp // 128
+        tiles = gl.nblocks * (nt * (nt + 1) // 2 if sym else nt * (lay.np_ // 128))
+        # 128-wide tiles from one per CU on, else 64-wide
+        return f"ns_f32<{stage}, {tp if stage == 3 else 'F32T'}, {2 if tiles >= 256 else 1}>"
     if kind == "syrk":
         return "ns_sym_bf16<0>"
     if kind == "poly":
@@ -190,8 +194,8 @@ def stage_exec_flops(kind, gl):
         up = (nt * (nt + 1) / 2) / (nt * nt)
         full = {"syrk": mp * mp * kx * up, "poly": mp ** 3 * up, "px": mp * mp * np_, "px_apply": mp * mp * np_}
         return 2.0 * full.get(kind, 0) * N
-    nt = mp // 256
-    sym = (nt * (nt - 1) / 2 + nt * 36 / 64) / (nt * nt)
+    side = [min(256, mp - i) for i in range(0, mp, 256)]   # the last tile may be partial
+    sym = ((mp * mp - sum(t * t for t in side)) / 2 + sum(t * (t + 32) / 2 for t in side)) / (mp * mp)
     kx = -(-lay.n // 32) * 32   # SYRK's K: n rounded up to the 32-deep slices
     if kind == "syrk":
         return 2.0 * mp * mp * kx * N * sym
@@ -702,7 +706,7 @@ def main():
     gbytes = torch.empty((), dtype=w.param_dtype).element_size()
     pack_b = sum(pack_bytes(gl, mom_bytes, gbytes, 4 if gl.struct.ns_dtype == 0 else 2)
                  for gl in opt._muon_planner.groups)
-    # Newton-Schulz in fp32 (the pretrain copy with fp32 momentum): priced against the fp32 MFMA peak
+    # Newton-Schulz in fp32 (the pretrain copy with fp32 momentum): priced at six bf16 products each
     ns32 = w.ns_dtype is None and w.momentum_dtype in (torch.float32, "fp8")
     peak = PEAK_F32_TFLOPS if ns32 else PEAK_BF16_TFLOPS
     res = {
@@ -717,7 +721,7 @@ def main():
                    "param_dtype": str(w.param_dtype).split(".")[-1],
                    "momentum_dtype": w.momentum_dtype if isinstance(w.momentum_dtype, str)
                    else str(w.momentum_dtype).split(".")[-1],
-                   "newton_schulz": ("fp32 MFMA" if ns32 else "bf16 MFMA, fp32 accumulate") + ", 5 iterations",
+                   "newton_schulz": ("fp32 as six bf16 MFMA products, fp32 accumulate" if ns32 else "bf16 MFMA, fp32 accumulate") + ", 5 iterations",
                    "ns_form": args.ns_form, "shared_launches": not args.separate_groups,
                    "groups": [f"{gl.rows}x{gl.cols}x{gl.nblocks}" for gl in opt._muon_planner.groups]},
         "median_event_ms": round(median_ms, 3),

@@ -17,7 +17,7 @@ from pathlib import Path
 
 import torch
 
-from bench import (PEAK_BF16_TFLOPS, PEAK_F32_TFLOPS, PEAK_HBM_GBS, ROOT, _ns_plan, build_gpu, kernel_symbol, log,
+from bench import (PEAK_BF16_TFLOPS, PEAK_HBM_GBS, ROOT, _ns_plan, build_gpu, kernel_symbol, log,
                    stage_exec_flops)
 
 
@@ -184,8 +184,8 @@ def stage_bytes(kind, gl):
         up = (nt * (nt + 1) / 2) / (nt * nt)
         full = {"syrk": mp * mp * kx * up, "poly": mp ** 3 * up, "px": mp * mp * np_, "px_apply": mp * mp * np_}
         return 2.0 * full.get(kind, 0) * N
-    nt = mp // 256
-    up = nt * (nt + 1) // 2 * 256 * 256 * 2
+    side = [min(256, mp - i) for i in range(0, mp, 256)]   # the last tile may be partial
+    up = mp * mp + sum(t * t for t in side)                  # bytes: half the square and half the diagonal tiles
     kx = -(-lay.n // 32) * 32
     xin = mp * kx * 2
     if kind == "syrk":
@@ -571,9 +571,8 @@ def mfma_summary(args):
     """MFMA utilisation per Newton-Schulz kernel, and the instruction mix of
     the streaming kernels, from rocprofv3 counter runs
     (``--mfma-summary OUT.json CSV...``): executed MFMA FLOP (SQ_INSTS_MFMA x
-    32768, every instruction of the bf16 kernels being
-    v_mfma_f32_32x32x16_bf16, x 4096 for the fp32 kernels' v_mfma_f32_32x32x2_f32;
-    SQ_INSTS_VALU_MFMA_MOPS_BF16 / _F32 x 512 where collected), the
+    32768, every instruction being v_mfma_f32_32x32x16_bf16;
+    SQ_INSTS_VALU_MFMA_MOPS_BF16 x 512 where collected), the
     GFX clock the counters imply (GRBM_GUI_ACTIVE / 8 XCDs / duration) and the
     MFMA busy fraction of all 1024 SIMDs' cycles (SQ_VALU_MFMA_BUSY_CYCLES /
     (GRBM_GUI_ACTIVE / 8 x 1024), rocprofv3's MfmaUtil).  For the pack, AdamW
@@ -589,23 +588,18 @@ def mfma_summary(args):
         secs = c["duration_ns"] * 1e-9
         rec = {"dispatches": c["dispatches"], "avg_ms": round(secs * 1e3, 4)}
         if k.startswith("ns_") and "SQ_INSTS_MFMA" in c:
-            # bf16 kernels: v_mfma_f32_32x32x16_bf16 (32768 FLOP, 1024 FLOP per
-            # SIMD cycle at peak); fp32 kernels: v_mfma_f32_32x32x2_f32 (4096
-            # FLOP, 64 per SIMD cycle)
-            f32 = k.startswith("ns_f32")
-            flop = c["SQ_INSTS_MFMA"] * (4096.0 if f32 else 32768.0)
-            peak = PEAK_F32_TFLOPS if f32 else PEAK_BF16_TFLOPS
+            # v_mfma_f32_32x32x16_bf16 throughout (32768 FLOP, 1024 FLOP per SIMD cycle at
+            # peak); the fp32 kernels run six of its products per fp32 product
+            flop = c["SQ_INSTS_MFMA"] * 32768.0
             rec.update({"exec_flop": flop, "exec_tflops": round(flop / secs / 1e12, 1),
-                        "exec_frac_peak": round(flop / secs / 1e12 / peak, 4)})
-            if "SQ_INSTS_VALU_MFMA_MOPS_BF16" in c and not f32:
+                        "exec_frac_peak": round(flop / secs / 1e12 / PEAK_BF16_TFLOPS, 4)})
+            if "SQ_INSTS_VALU_MFMA_MOPS_BF16" in c:
                 rec["mops_flop"] = c["SQ_INSTS_VALU_MFMA_MOPS_BF16"] * 512.0
-            if "SQ_INSTS_VALU_MFMA_MOPS_F32" in c and f32:
-                rec["mops_flop"] = c["SQ_INSTS_VALU_MFMA_MOPS_F32"] * 512.0
             if "GRBM_GUI_ACTIVE" in c:
                 cycles = c["GRBM_GUI_ACTIVE"] / XCDS
                 rec["gfx_mhz"] = round(cycles / secs / 1e6, 1)
                 # what the kernel executed against the peak at the clock it ran at
-                rec["exec_frac_at_clock"] = round(flop / (cycles * simds * (64.0 if f32 else 1024.0)), 4)
+                rec["exec_frac_at_clock"] = round(flop / (cycles * simds * 1024.0), 4)
                 if "SQ_VALU_MFMA_BUSY_CYCLES" in c:
                     rec["mfma_busy"] = round(c["SQ_VALU_MFMA_BUSY_CYCLES"] / (cycles * simds), 4)
         elif k.startswith(("ns_", "pack", "adamw", "fp8_", "block_scale", "zero_pads")) and "SQ_INSTS_VALU" in c:
