@@ -528,96 +528,140 @@ __global__ __launch_bounds__(GE::NTH, GE::PER_CU * GE::NW / 4) void butterfly_ge
 
 // ---------------------------------------------------------------------------
 // The forward products for a few tokens (generation): 16 features x 16 NT tokens per
-// workgroup, whose waves split K and add their fp32 partials in wave order.
+// workgroup, all of K.  LW waves load: they keep RING groups of U steps of 32 k in LDS;
+// NT waves multiply, one per token tile.
 //
-// Bound by the weights' read.  A 64-wide tile leaves most of the chip idle here (4 x
-// 1024 features are 64 workgroups) and walks all of K behind a barrier per slice; with
-// 16 features per workgroup and an eighth of K per wave, every wave streams its own
-// slices through its own ring, without barriers, and 256 workgroups have 24 KiB and
-// more in flight each.  Forward of the 6.89B up-projection at 1 / 8 / 32 / 64 tokens 26 / 26
-// / 26 / 27 -> 12 / 13 / 16 / 22 us, the 1.3B query 13.5 / 13.7 / 14 / 14 -> 6.6 / 7.0 /
-// 8.2 / 10.5, the toy up-projection 9.5 / 9.8 / 10.2 / 10.3 -> 6.0 / 6.2 / 6.6 / 7.9.
-// The slices go through LDS because fragment loads straight into registers put
-// neighbouring lanes in different rows: 64 tokens of the first 27 us.  Short rings: more
-// workgroups per CU are worth more than deeper ones (64 tokens: 25 us with 4 slots).
-// Each workgroup reads all tokens again, which is what grows with them; from 128 on
-// the tiles are as fast (28 us).
+// Each output is one chain of MFMAs over K in the order of the tiles above
+// (v_mfma_f32_16x16x32_bf16 gives the bits of two v_mfma_f32_32x32x16_bf16 in a row:
+// measured on 8192 sums of 1024 products), so a row does not depend on the number of
+// tokens that share its call.  Eight waves with an eighth of K each, their partials added
+// at the end, were no faster (below, in brackets) and gave other bits.
+//
+// A 64-wide tile leaves most of the chip idle here (4 x 1024 features are 64 workgroups),
+// and a wave issues a 1 KiB load in about 100 cycles, so the loads are spread over four
+// waves that do nothing else; the multiplying waves read a group while the products of
+// the one before run.  Forward in us at 1 / 8 / 32 / 64 tokens, tiles -> now [split K]:
+//   6.89B up     53 / 55 / 55 / 56 -> 7.5 / 8.0 / 11.3 / 16.2  [8.1 / 8.7 / 12.5 / 19.1]
+//   6.89B down   83 / 84 / 85 / 85 -> 7.7 / 8.1 / 10.3 / 14.7  [7.3 / 8.2 / 12.2 / 18.0]
+//   1.3B query   35 / 36 / 36 / 36 -> 5.1 / 5.5 /  6.2 /  7.6  [5.4 / 5.5 /  6.5 /  8.6]
+// (tiles: the 256-wide ones and the interleaving copy; the 64-wide tiles take 22.6, 30.9
+// and 12.6 us at 65 tokens).  With weights that come from HBM (a rotation through 512 MB)
+// the first takes 11.1 / 11.5 / 16.3 / 20.5 us, the second 11.8 / 12.2 / 14.6 / 18.9.
+// What bounds it: of the 8.0 us at 8 tokens, two dependent launches that fill and drain
+// take 4.9 (the toy up-projection, 1 MB of weights); the rest reads 31 MB of weights, at
+// 10 TB/s from the Infinity Cache or 4.7 from HBM.  Each workgroup reads all tokens again,
+// which is what grows with them.  A single wave that loads and multiplies took 9.1 and
+// 12.1 us (first and second at 8 tokens); groups of eight steps in three slots 9.8 and
+// 8.5; six slots 8.5 and 8.2, five with NT > 1 12.2 us at 32 tokens and 18.4 at 64 (fewer
+// workgroups per CU); eight loading waves 8.7 and 8.5.
 // ---------------------------------------------------------------------------
-constexpr int FEW_W = 8;        // waves of a workgroup, which share K
 constexpr int FEW_TOKENS = 64;  // largest number of tokens
 constexpr int FEW_K = 32;       // k of a step
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int NT, bool FEATURES>
-__global__ __launch_bounds__(64 * FEW_W) void butterfly_few(GemmArgs a) {
-  constexpr int RING = NT == 1 ? 3 : 2, DMA = 1 + NT;  // K steps in flight per wave, 1 KiB loads of a step
-  constexpr int LD = 20;  // floats per token of a staged partial (16 features; rows start on different banks)
-  constexpr int WLDS = RING * DMA * 1024, RED = FEW_W * NT * 16 * LD * 4;
-  __shared__ __attribute__((aligned(1024))) char lds[FEW_W * WLDS > RED ? FEW_W * WLDS : RED];
+template <int NT, int LW, int U, int RING, bool FEATURES>
+__global__ __launch_bounds__(64 * (LW + NT)) void butterfly_few(GemmArgs a) {
+  constexpr int TILES = 1 + NT;             // 1 KiB loads of a step: the features, the token tiles
+  constexpr int PW = U * TILES / LW;        // loads per loading wave and group
+  constexpr int GROUPB = U * TILES * 1024;  // LDS bytes of a group
+  static_assert(PW * LW == U * TILES && RING >= 2 && PW * RING <= 63, "whole loads per wave, counted by vmcnt");
+  __shared__ __attribute__((aligned(1024))) char lds[RING * GROUPB];
   const int g = blockIdx.x / a.tiles_n, n0 = (blockIdx.x % a.tiles_n) * 16;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const i32x4 wr = buffer_rsrc(a.b.base + int64_t(g) * a.b.bstride + n0 * a.b.mstride);
-  const i32x4 xr = buffer_rsrc(a.a.base + int64_t(g) * a.a.bstride);
-  // loads: row lane/4, 16-B chunk of the step's 64 B at (lane%4) ^ (row/4)%4
-  const int lrow = lane >> 2, lk = ((lane & 3) ^ ((lane >> 4) & 3)) * 8;
-  uint32_t ro[DMA];
-  ro[0] = n0 + lrow < a.N ? uint32_t(lrow * a.b.mstride) : OOB;
+  if (wave < LW) {
+    // load q of this wave in a group: load u = wave + LW q, tile u % TILES of step u / TILES.
+    // A lane loads row lane/4, 16-B chunk of the step's 64 B at (lane%4) ^ (row/4)%4.
+    const int lrow = lane >> 2, lk = ((lane & 3) ^ ((lane >> 4) & 3)) * 8;
+    const i32x4 wr = buffer_rsrc(a.b.base + int64_t(g) * a.b.bstride + n0 * a.b.mstride);
+    const i32x4 xr = buffer_rsrc(a.a.base + int64_t(g) * a.a.bstride);
+    uint32_t off[PW];  // lane offset in the group that starts at k = 0; OOB beyond M and N
+    int kq[PW];        // this lane's k within the group
 #pragma unroll
-  for (int t = 0; t < NT; ++t) ro[1 + t] = t * 16 + lrow < a.M ? uint32_t((t * 16 + lrow) * a.a.mstride) : OOB;
-  const int kbeg = wave * a.kchunk, kend = min(a.K, kbeg + a.kchunk);
-  char* const ring = lds + wave * WLDS;
-  const uint32_t ring0 = lds_addr(ring);
-  auto issue = [&](int k, int slot) {
-    const uint32_t ko = k + lk < kend ? uint32_t(k + lk) * 2 : OOB;
-#pragma unroll
-    for (int q = 0; q < DMA; ++q)
-      bdma16(q == 0 ? wr : xr, (ro[q] | ko) & OOB ? OOB : ro[q] + ko, ring0 + (slot * DMA + q) * 1024);
-  };
-  // fragments: row lane%16, k 8 (lane/16) .. +7
-  const int l16 = lane & 15;
-  const uint32_t frag = uint32_t(l16 * 64 + (((lane >> 4) ^ (l16 >> 2)) << 4));
-  f32x4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f32x4{};
-  if (kbeg < kend) {
-#pragma unroll
-    for (int q = 0; q < RING; ++q) issue(kbeg + FEW_K * q, q);
-    int slot = 0;
-    for (int k = kbeg; k < kend; k += FEW_K) {
-      wait_vm<(RING - 1) * DMA>();
-      const char* s = ring + slot * DMA * 1024 + frag;
-      const bf16x8 w = *reinterpret_cast<const bf16x8*>(s);
-      bf16x8 x[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) x[t] = *reinterpret_cast<const bf16x8*>(s + (1 + t) * 1024);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the slot is loaded again
-      issue(k + FEW_K * RING, slot);
-      slot = slot + 1 == RING ? 0 : slot + 1;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[t], acc[t], 0, 0, 0);
+    for (int q = 0; q < PW; ++q) {
+      const int u = wave + LW * q, tile = u % TILES, row = (tile == 0 ? 0 : (tile - 1) * 16) + lrow;
+      kq[q] = (u / TILES) * FEW_K + lk;
+      const bool in = tile == 0 ? n0 + lrow < a.N : row < a.M;
+      off[q] = in ? uint32_t(row * (tile == 0 ? a.b.mstride : a.a.mstride)) + kq[q] * 2 : OOB;
     }
-    wait_vm<0>();
+    const uint32_t lds0 = lds_addr(lds) + wave * 1024;
+    // the group that starts at k; beyond K it loads zeros
+    auto issue = [&](int k, int slot) {
+#pragma unroll
+      for (int q = 0; q < PW; ++q) {
+        const int u = wave + LW * q;
+        const bool in = off[q] != OOB && k + kq[q] < a.K;
+        bdma16(u % TILES == 0 ? wr : xr, in ? off[q] + uint32_t(k) * 2 : OOB, lds0 + slot * GROUPB + LW * q * 1024);
+      }
+    };
+#pragma unroll
+    for (int r = 0; r < RING - 1; ++r) issue(FEW_K * U * r, r);
+    int slot = RING - 1;
+    for (int k = 0; k < a.K; k += FEW_K * U) {
+      wait_vm<(RING - 2) * PW>();  // this wave's loads of the group landed
+      barrier();                   // every wave's, and the group before is read
+      issue(k + FEW_K * U * (RING - 1), slot);
+      slot = slot + 1 == RING ? 0 : slot + 1;
+    }
+    wait_vm<0>();  // no load is left in flight to LDS that another workgroup may own next
+    return;
   }
-  __syncthreads();
-  // lane: token l16, features 4 (lane/16) .. +3
-  float* red = reinterpret_cast<float*>(lds);
+  const int tile = wave - LW, l16 = lane & 15;
+  // fragments: row lane%16, k 8 (lane/16) .. +7
+  const char* const frag = lds + l16 * 64 + (((lane >> 4) ^ (l16 >> 2)) << 4);
+  struct Fr {
+    bf16x8 w[U], x[U];
+  };
+  f32x4 acc = {};
+  int k = 0, slot = 0;
+  auto read = [&](Fr& f) {  // the group that the barrier just completed
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-    *reinterpret_cast<f32x4*>(red + ((wave * NT + t) * 16 + l16) * LD + (lane >> 4) * 4) = acc[t];
-  __syncthreads();
-  for (int i = threadIdx.x; i < NT * 256; i += 64 * FEW_W) {
-    const int f = i & 15, tok = i >> 4, col = n0 + f;
-    float v = 0.f;
+    for (int u = 0; u < U; ++u) {
+      const char* s = frag + slot * GROUPB + u * TILES * 1024;
+      f.w[u] = *reinterpret_cast<const bf16x8*>(s);
+      f.x[u] = *reinterpret_cast<const bf16x8*>(s + (1 + tile) * 1024);
+    }
+    slot = slot + 1 == RING ? 0 : slot + 1;
+    k += FEW_K * U;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto mul = [&](const Fr& f) {
 #pragma unroll
-    for (int w = 0; w < FEW_W; ++w) v += red[(w * NT * 16 + tok) * LD + f];
-    if (tok >= a.M || col >= a.N) continue;
-    char* dst = a.c.base + int64_t(tok) * a.c.rstride;
-    if (FEATURES)
-      dst += (int64_t(col) * a.G + g) * 2;
-    else
-      dst += int64_t(g) * a.c.bstride + (col & ((1 << a.c.log2l) - 1)) * a.c.cplane + int64_t(col >> a.c.log2l) * 2;
-    *reinterpret_cast<uint16_t*>(dst) = f2bf(v);
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.x[u], f.w[u], acc, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto next_group = [&] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this group is read: its slot may be loaded again
+    barrier();
+  };
+  Fr fa, fb;
+  barrier();
+  read(fa);
+  while (k < a.K) {
+    next_group();
+    read(fb);
+    mul(fa);
+    if (k >= a.K) {
+      fa = fb;
+      break;
+    }
+    next_group();
+    read(fa);
+    mul(fb);
+  }
+  mul(fa);
+  // lane: feature l16, tokens 4 (lane/16) .. +3 of the wave's token tile
+  const int col = n0 + l16;
+  if (col >= a.N) return;
+  char* dst = a.c.base;
+  if (FEATURES)
+    dst += (int64_t(col) * a.G + g) * 2;
+  else
+    dst += int64_t(g) * a.c.bstride + (col & ((1 << a.c.log2l) - 1)) * a.c.cplane + int64_t(col >> a.c.log2l) * 2;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int tok = tile * 16 + (lane >> 4) * 4 + e;
+    if (tok < a.M) *reinterpret_cast<uint16_t*>(dst + int64_t(tok) * a.c.rstride) = f2bf(acc[e]);
   }
 }
 
@@ -798,14 +842,18 @@ void launch_gemm_t(const GemmArgs& a, hipStream_t s) {
   else launch_gemm_g<G64, AT, BT, OUT>(a, s);
 }
 
+template <int NT, int RING, bool FEATURES>
+void launch_few_t(const GemmArgs& a, hipStream_t s) {
+  constexpr int LW = 4, U = 4;
+  const dim3 grid(unsigned(a.G * a.tiles_n)), block(64 * (LW + NT));
+  hipLaunchKernelGGL((butterfly_few<NT, LW, U, RING, FEATURES>), grid, block, 0, s, a);
+}
 template <bool FEATURES>
 void launch_few(GemmArgs a, hipStream_t s) {
   a.tiles_n = cdiv(a.N, 16);
-  a.kchunk = cdiv(a.K, FEW_K * FEW_W) * FEW_K;
-  const dim3 grid(unsigned(a.G * a.tiles_n)), block(64 * FEW_W);
-  if (a.M <= 16) hipLaunchKernelGGL((butterfly_few<1, FEATURES>), grid, block, 0, s, a);
-  else if (a.M <= 32) hipLaunchKernelGGL((butterfly_few<2, FEATURES>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((butterfly_few<4, FEATURES>), grid, block, 0, s, a);
+  if (a.M <= 16) launch_few_t<1, 5, FEATURES>(a, s);
+  else if (a.M <= 32) launch_few_t<2, 4, FEATURES>(a, s);
+  else launch_few_t<4, 4, FEATURES>(a, s);
 }
 
 void launch_reduce(const GemmArgs& a, const GOut& c, hipStream_t s) {

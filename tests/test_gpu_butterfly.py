@@ -132,6 +132,26 @@ def test_forward_for_few_tokens(tokens, dims):
     assert torch.equal(y, out.transpose(1, 2).reshape(tokens, s * nb))
 
 
+# token counts on both sides of every switch of kernel and tile width: 16 / 32 / 64 tokens per workgroup, 64-, 128- and
+# 256-wide tiles (the largest count takes the 256-wide ones); K in whole slices and ending inside one
+@pytest.mark.parametrize("dims", [(4, 512, 512, 512), (2, 512, 1096, 264), (1, 1024, 2744, 520), (16, 512, 264, 56)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_rows_do_not_depend_on_the_token_count(dims):
+    """A row of the forward and of dx is the same, bit for bit, whatever number of tokens shares its call."""
+    print("rows", dims, flush=True)
+    nb, q, p, s = dims
+    x, w1, w2, dout = gpu(*make(16384, nb, q, p, s, seed=11))
+    out, out1 = butterfly_blk_op(x, w1, w2)
+    y = butterfly_blk(x, w1, w2)
+    dx = butterfly_blk_bwd_op(x, w1, w2, out1, dout)[0]
+    for n in (1, 8, 16, 17, 32, 33, 64, 65, 128, 300, 1000, 2000, 4096):
+        print("  tokens", n, flush=True)
+        o, o1 = butterfly_blk_op(x[:n], w1, w2)
+        assert torch.equal(o1, out1[:, :n]) and torch.equal(o, out[:n]), n
+        assert torch.equal(butterfly_blk(x[:n], w1, w2), y[:n]), n
+        assert torch.equal(butterfly_blk_bwd_op(x[:n], w1, w2, o1, dout[:n])[0], dx[:n]), n
+
+
 @pytest.mark.parametrize("how", ["compile", "saved_hooks", "expanded_grad", "second_order"])
 def test_layer_operator_under_torch(how):
     """The native operator traced by torch.compile, with saved-tensor hooks and with a gradient that is no dense
