@@ -71,6 +71,13 @@ mmuon_butterfly_args make_args(const Tensor& x2, const Tensor& w1, const Tensor&
   return a;
 }
 
+// The kernels read rows of 16-B chunks.  A gradient may be a contiguous view at any element
+// (one of the parts that torch.cat's backward hands out): such a one is copied.
+Tensor dense_aligned(const Tensor& t) {
+  const Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.const_data_ptr()) % 16 == 0 ? c : c.clone();
+}
+
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 Pair linear_impl(const Tensor& x, const Tensor& w1_, const Tensor& w2_) {
@@ -88,7 +95,7 @@ Pair linear_impl(const Tensor& x, const Tensor& w1_, const Tensor& w2_) {
 Triple linear_bwd_impl(const Tensor& x, const Tensor& w1_, const Tensor& w2_, const Tensor& out1_,
                        const Tensor& dout_) {
   const Tensor x2 = x.contiguous(), w1 = w1_.contiguous(), w2 = w2_.contiguous();
-  const Tensor out1 = out1_.contiguous(), dout = dout_.contiguous();
+  const Tensor out1 = out1_.contiguous(), dout = dense_aligned(dout_);
   mmuon_butterfly_args a = make_args(x2, w1, w2);
   TORCH_CHECK_VALUE(out1.dim() == 3 && out1.size(0) == w2.size(0) && out1.size(1) == x2.size(0) &&
                         out1.size(2) == w2.size(2) && dout.dim() == 2 && dout.size(0) == x2.size(0) &&

@@ -176,6 +176,20 @@ def test_layer_operator_under_torch(how):
     assert torch.equal(y, z) and all(torch.equal(u, v) for u, v in zip(got, want))
 
 
+@pytest.mark.parametrize("start", [1, 3, 7])
+def test_gradient_that_starts_anywhere(start):
+    """A gradient that is a contiguous view ``start`` elements into its storage, as torch.cat's backward hands out."""
+    x, w1, w2, _ = gpu(*make(96, 2, 64, 64, 72, seed=4))
+    a, b = ([t.clone().requires_grad_() for t in (x, w1, w2)] for _ in range(2))
+    y = butterfly_blk(*a)
+    dy = torch.randn(y.shape, generator=torch.Generator().manual_seed(1)).to(DEV, torch.bfloat16)
+    want = torch.autograd.grad(y, a, dy)
+    head = torch.zeros(start, dtype=torch.bfloat16, device=DEV)
+    z = torch.cat([head, butterfly_blk(*b).flatten()])
+    got = torch.autograd.grad(z, b, torch.cat([head, dy.flatten()]))
+    assert all(torch.equal(u, v) for u, v in zip(got, want))
+
+
 def test_gradient_through_the_intermediate_alone_is_zero():
     """out1 carries no gradient of its own; asking for one through it alone gives zeros."""
     x, w1, w2, _ = gpu(*make(64, 2, 64, 64, 64))
