@@ -393,8 +393,8 @@ size_t mmuon_butterfly_linear_workspace(const mmuon_butterfly_args* a);
 /* Thread-local message of the last failing call ("" if none). */
 const char* mmuon_last_error(void);
 
-/* ABI version: bumped when a declaration of this header changes (not when one
-   is added). */
+/* ABI version: bumped on any change to this header. */
+#define MMUON_ABI_VERSION 8
 int mmuon_abi_version(void);
 
 #ifdef __cplusplus

@@ -12,13 +12,16 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(os.environ.get("MMUON_LIB", Path(__file__).resolve().parent / "libmmuon.so"))
+ABI_VERSION = 8
+# the layer's torch operator; the name carries the ABI, so that one built for another is never loaded (once loaded,
+# its registrations stay for the life of the process)
+TORCH_LIB_PATH = Path(__file__).resolve().parent / f"libmmuon_torch.{ABI_VERSION}.so"
 
 F32, BF16, F8E4M3, F8E5M2 = 0, 1, 2, 3
 GROUP_ALIGNED16 = 1
 NS_NO_APPLY = 1
 NS_STANDARD = 2
 NS_HOLD_LAST = 4
-ABI_VERSION = 7
 # Newton-Schulz plan ops (MMUON_NSOP_*) and buffers (MMUON_NSB_*)
 NSOP_SYRK, NSOP_POLY, NSOP_PX, NSOP_PX_APPLY, NSOP_SYMM = 0, 1, 2, 3, 4
 NSB_X0, NSB_X1, NSB_A, NSB_P, NSB_X0_S0, NSB_X0_S1, NSB_X1_S0, NSB_X1_S1, NSB_PARAM = range(9)
@@ -147,12 +150,17 @@ def lib() -> C.CDLL:
                 f"{LIB_PATH} is missing: build it with `python -m monarch_muon_amd.build` "
                 "(the MI355X kernels have no fallback)")
         handle = C.CDLL(str(LIB_PATH))
-        for name, (res, args) in SIGNATURES.items():
-            fn = getattr(handle, name)
-            fn.restype = res
-            fn.argtypes = args
-        if handle.mmuon_abi_version() != ABI_VERSION:
-            raise RuntimeError(f"{LIB_PATH} has ABI {handle.mmuon_abi_version()}, expected {ABI_VERSION}")
+        try:
+            found = handle.mmuon_abi_version()
+            if found != ABI_VERSION:
+                raise RuntimeError(f"{LIB_PATH} has ABI {found}, expected {ABI_VERSION}: build it again with "
+                                   "`python -m monarch_muon_amd.build`")
+            for name, (res, args) in SIGNATURES.items():
+                fn = getattr(handle, name)
+                fn.restype = res
+                fn.argtypes = args
+        except AttributeError as e:
+            raise RuntimeError(f"{LIB_PATH} lacks a function of ABI {ABI_VERSION}: {e}") from None
         _lib = handle
     return _lib
 

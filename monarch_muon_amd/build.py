@@ -2,7 +2,7 @@
 
 ``python -m monarch_muon_amd.build`` compiles every ``csrc/*.hip`` to an object
 in parallel and links the shared library next to this file, and beside it
-``libmmuon_torch.so``, the layer's native torch operator (``csrc/torch_ops.cpp``,
+``libmmuon_torch.<ABI>.so``, the layer's native torch operator (``csrc/torch_ops.cpp``,
 host code only).  hipcc cross-compiles for gfx950 without a GPU.  ``build_probe()`` builds the
 bench-only HBM streaming probe (``bench_probe.hip`` beside ``bench.py``) into a
 library of its own, apart from the optimizer's.
@@ -16,10 +16,11 @@ import subprocess
 import sys
 from pathlib import Path
 
+from ._abi import TORCH_LIB_PATH as TORCH_LIB
+
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libmmuon.so"
-TORCH_LIB = HERE / "libmmuon_torch.so"
 ARCH = "gfx950"
 
 CFLAGS = [
@@ -63,6 +64,9 @@ def _build_torch_ops() -> None:
     if r.returncode != 0:
         raise RuntimeError(f"torch_ops.cpp failed:\n{r.stdout}{r.stderr}")
     os.replace(tmp, TORCH_LIB)
+    for old in HERE.glob("libmmuon_torch*.so"):   # built for another ABI: never loaded again
+        if old != TORCH_LIB:
+            old.unlink()
 
 
 def build(verbose: bool = True) -> Path:

@@ -20,7 +20,6 @@ the reference's models satisfies.  Other inputs raise; there is no fallback.
 from __future__ import annotations
 
 import ctypes as C
-from pathlib import Path
 
 import torch
 
@@ -129,18 +128,34 @@ butterfly_blk_op.register_autograd(_backward, setup_context=_setup_context)
 # The layer's own form of the pair, ``mmuon::butterfly_linear`` and ``mmuon::butterfly_linear_bwd``
 # (csrc/torch_ops.cpp, autograd included): output and its gradient in feature order, (B, s l) with
 # feature j l + ll the column j of block ll, so no interleaving pass follows the products.
-_TORCH_LIB = Path(__file__).resolve().parent / "libmmuon_torch.so"
+# Importing registers the operator if it has been built; the kernels' library is loaded by the
+# operator's first launch (_bind), so a process may build it, or name another, after the import.
 _BOUND = ("mmuon_butterfly_linear_fwd", "mmuon_butterfly_linear_bwd", "mmuon_butterfly_linear_workspace",
           "mmuon_last_error")
+_linear_op = _torch_lib = None
 
 
-def _load_linear():
-    """The native operator, bound to the library ``_abi`` loads; raises where either is missing."""
-    lib = _abi.lib()
-    if not _TORCH_LIB.exists():
-        raise RuntimeError(f"{_TORCH_LIB} is missing: build it with `python -m monarch_muon_amd.build`")
-    torch.ops.load_library(str(_TORCH_LIB))
-    C.CDLL(str(_TORCH_LIB)).mmuon_torch_bind(*(C.cast(getattr(lib, name), C.c_void_p) for name in _BOUND))
+@C.CFUNCTYPE(C.c_int)
+def _bind() -> int:
+    """Give the operator the functions of the library that ``_abi`` loads (called by the operator, any thread)."""
+    try:
+        lib = _abi.lib()
+        return _torch_lib.mmuon_torch_bind(lib.mmuon_abi_version(),
+                                           *(C.cast(getattr(lib, name), C.c_void_p) for name in _BOUND))
+    except Exception as e:
+        _torch_lib.mmuon_torch_refuse(str(e).encode())
+        return -1
+
+
+def _load_linear() -> None:
+    """Register the native operator; raises where it is not built."""
+    global _linear_op, _torch_lib
+    path = _abi.TORCH_LIB_PATH
+    if not path.exists():
+        raise RuntimeError(f"{path} is missing: build it with `python -m monarch_muon_amd.build`")
+    torch.ops.load_library(str(path))
+    _torch_lib = C.CDLL(str(path))
+    _torch_lib.mmuon_torch_set_loader(_bind)
 
     @torch.library.register_fake("mmuon::butterfly_linear")
     def _(x2, w1, w2):
@@ -149,13 +164,13 @@ def _load_linear():
         return x2.new_empty(B, s * l), x2.new_empty(l, B, r)
 
     torch.library.register_fake("mmuon::butterfly_linear_bwd", _bwd_fake)
-    return torch.ops.mmuon.butterfly_linear.default
+    _linear_op = torch.ops.mmuon.butterfly_linear.default
 
 
 try:
-    _linear_op = _load_linear()
-except (RuntimeError, OSError) as e:   # not built: the first call raises
-    _linear_op, _linear_error = None, e
+    _load_linear()
+except (RuntimeError, OSError):   # not built yet: butterfly_blk tries again and raises
+    pass
 
 
 def butterfly_blk(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> torch.Tensor:
@@ -164,7 +179,7 @@ def butterfly_blk(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> torch.
         dt = torch.get_autocast_dtype("cuda")
         x, w1, w2 = x.to(dt), w1.to(dt), w2.to(dt)
     if _linear_op is None:
-        raise RuntimeError(str(_linear_error))
+        _load_linear()
     if x.dim() == 2:
         return _linear_op(x, w1, w2)[0]
     batch_shape, n = x.shape[:-1], x.shape[-1]

@@ -7,8 +7,9 @@
 // dispatches, ctypes calls) took 190 us of host time, so the GPU waited for the host up
 // to about 4000 tokens of the 1.3B layers.
 //
-// The library's functions are bound at run time (mmuon_torch_bind) to the ones that
-// monarch_muon_amd/_abi.py has loaded, so MMUON_LIB selects them here too.
+// The library's functions are bound at the first launch (loader, mmuon_torch_bind) to the
+// ones that monarch_muon_amd/_abi.py loads, so MMUON_LIB selects them here too; a library of
+// another ABI than this file was compiled with is refused.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -16,6 +17,9 @@
 #include <torch/library.h>
 
 #include <algorithm>
+#include <atomic>
+#include <mutex>
+#include <string>
 #include <tuple>
 
 #include "../../include/mmuon.h"
@@ -32,6 +36,15 @@ struct Abi {
   size_t (*workspace)(const mmuon_butterfly_args*) = nullptr;
   const char* (*last_error)() = nullptr;
 } abi;
+std::atomic<bool> bound{false};
+int (*loader)() = nullptr;         // loads the library and binds it; 0 where it did
+thread_local std::string refusal;  // why it did not
+
+void bind_library() {
+  if (bound.load(std::memory_order_acquire)) return;
+  refusal = "libmmuon.so is not loaded";
+  TORCH_CHECK(loader != nullptr && loader() == 0, refusal);
+}
 
 void check_rc(int rc, const char* what) {
   TORCH_CHECK(rc == 0, what, " failed (code ", rc, "): ", abi.last_error());
@@ -42,7 +55,6 @@ void require_cuda(const Tensor& t) {
 }
 
 mmuon_butterfly_args make_args(const Tensor& x2, const Tensor& w1, const Tensor& w2) {
-  TORCH_CHECK(abi.fwd != nullptr, "libmmuon.so is not loaded");
   for (const Tensor* t : {&x2, &w1, &w2}) require_cuda(*t);
   const char* names[3] = {"x", "w1", "w2"};
   const Tensor* ts[3] = {&x2, &w1, &w2};
@@ -58,6 +70,7 @@ mmuon_butterfly_args make_args(const Tensor& x2, const Tensor& w1, const Tensor&
   // 32-bit sides in the C struct; the library checks their ranges
   TORCH_CHECK_VALUE(std::max({w1.size(0), w1.size(1), w1.size(2), w2.size(1)}) <= INT32_MAX,
                     "butterfly: block sides beyond 32 bits");
+  bind_library();
   mmuon_butterfly_args a{};
   a.tokens = x2.size(0);
   a.nblocks = int32_t(w1.size(0));
@@ -208,9 +221,27 @@ TORCH_LIBRARY_IMPL(mmuon, Autograd, m) {
   m.impl("butterfly_linear_bwd", linear_bwd_autograd);
 }
 
-extern "C" void mmuon_torch_bind(void* fwd, void* bwd, void* workspace, void* last_error) {
+extern "C" {
+
+void mmuon_torch_set_loader(int (*fn)()) { loader = fn; }
+
+void mmuon_torch_refuse(const char* why) { refusal = why; }
+
+int mmuon_torch_bind(int version, void* fwd, void* bwd, void* workspace, void* last_error) {
+  if (version != MMUON_ABI_VERSION) {
+    refusal = "the layer's operator was built for ABI " + std::to_string(MMUON_ABI_VERSION) + ", libmmuon.so has ABI " +
+              std::to_string(version) + ": build both again with `python -m monarch_muon_amd.build`";
+    return -1;
+  }
+  static std::mutex mutex;
+  const std::lock_guard<std::mutex> lock(mutex);
+  if (bound) return 0;  // by another thread's first call
   abi.fwd = reinterpret_cast<decltype(abi.fwd)>(fwd);
   abi.bwd = reinterpret_cast<decltype(abi.bwd)>(bwd);
   abi.workspace = reinterpret_cast<decltype(abi.workspace)>(workspace);
   abi.last_error = reinterpret_cast<decltype(abi.last_error)>(last_error);
+  bound.store(true, std::memory_order_release);
+  return 0;
 }
+
+}  // extern "C"
