@@ -559,6 +559,7 @@ __device__ __forceinline__ void stage_tile(char* stage, const f32x16 (&acc)[TMI]
 // T[r][i] for the BN staged rows, dst at the first staged row of the tile's
 // first column panel (panel stride pstride).  One wave instruction writes rows
 // 16u .. 16u+15 of one panel (1 KiB contiguous).
+template <bool PART>
 __device__ __forceinline__ void stage_rows(const char* stage, uint16_t* dst, int64_t pstride, int rows) {
   const int tid = fresh_tid();
   const int lane = tid & 63, wave = tid >> 6;
@@ -567,7 +568,7 @@ __device__ __forceinline__ void stage_rows(const char* stage, uint16_t* dst, int
     const int u = wave + NWAVES * it;  // 8 panels x BN/16 row blocks
     const int q = u & 7, r = (u >> 3) * 16 + (lane >> 2);
     const int i = q * 32 + (lane & 3) * 8;
-    if (i >= rows || r >= rows) continue;  // beyond a partial tile
+    if (PART && (i >= rows || r >= rows)) continue;  // beyond a partial tile
     const uint4 v = *reinterpret_cast<const uint4*>(stage + tile_off(r, i));
     *reinterpret_cast<uint4*>(dst + q * pstride + r * PANEL + (lane & 3) * 8) = v;
   }
@@ -612,7 +613,9 @@ __device__ __forceinline__ void stage_cols(const char* stage, Fn&& fn) {
 // ---------------------------------------------------------------------------
 static_assert(BM == BN, "square tiles: a symmetric tile is either diagonal or strictly upper");
 // PART: the stacks' extents are no multiples of the tile, so tiles at their ends are
-// partial; without it those checks are constants (they cost the 1024 x 1024 blocks 1%).
+// partial; without it those checks are compiled out, of the stores too, where the compiler
+// cannot see that a lane's row lies in a whole tile (loads and waves' windows cost the
+// 1024 x 1024 blocks 1%, the stores SYRK 0.4%: 41 branches in its epilogue).
 template <int STAGE, bool PART>
 __device__ __forceinline__ void sym_work(const NsArgs& a, uint16_t* lds, int v) {
   const int nt = tiles_of(a.mp), nc = nt;
@@ -668,11 +671,11 @@ __device__ __forceinline__ void sym_work(const NsArgs& a, uint16_t* lds, int v) 
     // upper tile C[r0 + i][c0 + r] = T[r][i]
     uint16_t* dst = out + (c0 / PANEL) * pstride + int64_t(r0) * PANEL;
     stage_cols(stage, [&](int i, int r, const uint4& u) {
-      if (i < rows && r < cols) *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
+      if (!PART || (i < rows && r < cols)) *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
     });
   } else {
     // diagonal tile in full, through its mirror C[r0 + r][r0 + i] = T[r][i]
-    stage_rows(stage, out + (r0 / PANEL) * pstride + int64_t(r0) * PANEL, pstride, rows);
+    stage_rows<PART>(stage, out + (r0 / PANEL) * pstride + int64_t(r0) * PANEL, pstride, rows);
   }
 }
 
@@ -813,7 +816,7 @@ __device__ __forceinline__ void px_work(const NsArgs& a, uint16_t* lds, int v) {
     uint16_t* dst = static_cast<uint16_t*>(a.out) + int64_t(b) * a.mp * a.np + (c0 / PANEL) * pstride +
                     int64_t(r0) * PANEL;
     stage_cols(stage, [&](int i, int r, const uint4& u) {
-      if (i < rows && r < cols) *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
+      if (!PART || (i < rows && r < cols)) *reinterpret_cast<uint4*>(dst + (r >> 5) * pstride + i * PANEL + (r & 31)) = u;
     });
     return;
   }
