@@ -143,27 +143,34 @@ OP_KIND = {0: "syrk", 1: "poly", 2: "px", 3: "px_apply", 4: "symm"}
 NS_KINDS = ("syrk", "poly", "symm", "px", "px_apply")
 
 
+def f32_tile(kind, gl):
+    """Tile side of an fp32 Newton-Schulz launch: 128 from one such tile per CU on, else 64."""
+    lay = gl.ws.layout
+    nt = lay.mp // 128
+    tiles = gl.nblocks * (nt * (nt + 1) // 2 if kind in ("syrk", "poly") else nt * (lay.np_ // 128))
+    return 128 if tiles >= 256 else 64
+
+
+def partial_tiles(kind, gl):
+    """Whether a bf16 Newton-Schulz launch runs the kernel whose last 256-wide tiles may be partial."""
+    lay = gl.ws.layout
+    return lay.mp % 256 != 0 or (kind in ("px", "px_apply") and lay.np_ % 256 != 0)
+
+
 def kernel_symbol(kind, gl, it, fp8=False):
     """The kernel (template instance) rocprof reports for a launch, as it
     appears in ``rocprofv3 --stats`` names (mmuon::(anonymous namespace)::...)."""
     tp = "BF16T" if gl is not None and gl.struct.param_dtype == 1 else "F32T"
     if gl is not None and kind in NS_KINDS and gl.struct.ns_dtype == 0:  # fp32 Newton-Schulz
         stage = {"syrk": 0, "poly": 1, "px": 2, "px_apply": 3}[kind]
-        lay, sym = gl.ws.layout, stage < 2
-        nt = lay.mp // 128
-        tiles = gl.nblocks * (nt * (nt + 1) // 2 if sym else nt * (lay.np_ // 128))
-        # 128-wide tiles from one per CU on, else 64-wide
-        return f"ns_f32<{stage}, {tp if stage == 3 else 'F32T'}, {2 if tiles >= 256 else 1}>"
-    if kind == "syrk":
-        return "ns_sym_bf16<0>"
-    if kind == "poly":
-        return "ns_sym_bf16<1>"
-    if kind == "symm":
-        return "ns_sym_bf16<4>"
-    if kind == "px":
-        return "ns_px_bf16<2, false, BF16T>"
-    if kind == "px_apply":
-        return f"ns_px_bf16<3, {'true' if gl.transposed else 'false'}, {tp}>"
+        return f"ns_f32<{stage}, {tp if stage == 3 else 'F32T'}, {f32_tile(kind, gl) // 64}>"
+    if gl is not None and kind in NS_KINDS:
+        edge = "edge_" if partial_tiles(kind, gl) else ""
+        if kind in ("syrk", "poly", "symm"):
+            return f"ns_sym_{edge}bf16<{ {'syrk': 0, 'poly': 1, 'symm': 4}[kind]}>"
+        if kind == "px":
+            return f"ns_px_{edge}bf16<2, false, BF16T>"
+        return f"ns_px_{edge}bf16<3, {'true' if gl.transposed else 'false'}, {tp}>"
     if kind == "pack":
         return ("fp8_" if fp8 else "") + ("pack_cols_kernel" if gl.transposed else "pack_rows_kernel")
     return kind + ("_fp8_kernel" if fp8 else "_kernel")
@@ -183,27 +190,33 @@ def stage_flops(kind, gl):
 
 
 def stage_exec_flops(kind, gl):
-    """MFMA FLOPs the kernels execute (padded tiles; symmetric stages compute the
-    256x256 tiles above the diagonal, and on a diagonal tile the 36 of its 64
-    32x32 MFMA tiles on or above the diagonal)."""
+    """MFMA FLOPs the kernels execute, fp32 products counted once (each is six of
+    bf16).  bf16: 256x256 tiles, each eight 128x64 windows; a window that lies in
+    the padding is left out (the columns' in PX, both where tiles may be partial).
+    Symmetric stages compute the tiles above the diagonal, and on a diagonal tile
+    the 32x32 MFMA tiles on or above the diagonal (36 of its 64).  fp32: 128- or
+    64-wide tiles without those in the padding, the upper ones of SYRK and POLY."""
+    if kind not in NS_KINDS:
+        return 0.0
     lay = gl.ws.layout
-    N, mp, np_ = gl.nblocks, lay.mp, lay.np_
-    if gl.struct.ns_dtype == 0:   # fp32 kernels: 128 x 128 tiles, SYRK / POLY the upper ones only
-        kx = -(-lay.n // 32) * 32   # SYRK's K: n rounded up to the 32-deep K tiles
-        nt = mp // 128
-        up = (nt * (nt + 1) / 2) / (nt * nt)
-        full = {"syrk": mp * mp * kx * up, "poly": mp ** 3 * up, "px": mp * mp * np_, "px_apply": mp * mp * np_}
-        return 2.0 * full.get(kind, 0) * N
-    side = [min(256, mp - i) for i in range(0, mp, 256)]   # the last tile may be partial
-    sym = ((mp * mp - sum(t * t for t in side)) / 2 + sum(t * (t + 32) / 2 for t in side)) / (mp * mp)
-    kx = -(-lay.n // 32) * 32   # SYRK's K: n rounded up to the 32-deep slices
-    if kind == "syrk":
-        return 2.0 * mp * mp * kx * N * sym
-    if kind in ("poly", "symm"):
-        return 2.0 * mp * mp * mp * N * sym
-    if kind in ("px", "px_apply"):
-        return 2.0 * mp * mp * np_ * N
-    return 0.0
+    m, n, sym = lay.m, lay.n, kind in ("syrk", "poly", "symm")
+    up = lambda x, unit: -(-x // unit) * unit
+    if gl.struct.ns_dtype == 0:
+        t = f32_tile(kind, gl)
+        rt, ct = -(-m // t), -(-n // t)
+        tiles = rt * (rt + 1) // 2 if sym else rt * ct
+        return 2.0 * t * t * up(n if kind == "syrk" else m, 16) * tiles * gl.nblocks
+    part = partial_tiles(kind, gl)
+    valid = m if sym else n   # of the columns
+    rows = [up(min(256, m - r), 128) if part else 256 for r in range(0, lay.mp, 256)]
+    cols = [up(max(0, min(256, valid - c)), 64) if part or not sym else 256
+            for c in range(0, lay.mp if sym else lay.np_, 256)]
+    if sym:
+        out = sum(rows[i] * cols[j] for i in range(len(rows)) for j in range(i + 1, len(cols)))
+        out += sum(1024 for r, c in zip(rows, cols) for i in range(r // 32) for j in range(i, 8) if 32 * j < c)
+    else:
+        out = sum(rows) * sum(cols)
+    return 2.0 * out * (up(n, 32) if kind == "syrk" else lay.mp) * gl.nblocks
 
 
 def _ns_plan(gl, opt):
@@ -358,21 +371,23 @@ def butterfly_flops(x, w1, w2):
 
 def torch_reference_fwd(x2, w1, w2):
     """pretrain/src/models/monarch/monarch_ops.py:23-36 with the eager riffle (right operands made
-    contiguous: transposed bf16 bmm operands are avoided on this platform)."""
+    contiguous: transposed bf16 bmm operands are avoided on this platform), and the output in
+    feature order (:105-114)."""
     B = x2.shape[0]
     k, q, p = w1.shape
     l, s, r = w2.shape
     out1 = torch.bmm(x2.reshape(B, k, p).transpose(0, 1), w1.transpose(-1, -2).contiguous())
     t = out1.transpose(0, 1).reshape(B, r, l).permute(2, 0, 1).contiguous()
-    return torch.bmm(t, w2.transpose(-1, -2).contiguous()).transpose(0, 1).contiguous(), t
+    out_blk = torch.bmm(t, w2.transpose(-1, -2).contiguous()).transpose(0, 1).contiguous()
+    return out_blk.transpose(1, 2).reshape(B, s * l), t
 
 
-def torch_reference_bwd(x2, w1, w2, out1, dout_blk):
-    """monarch_ops.py:57-82 with the eager unriffle."""
+def torch_reference_bwd(x2, w1, w2, out1, dy):
+    """monarch_ops.py:57-82 with the eager unriffle, from the gradient in feature order."""
     B = x2.shape[0]
     k, q, p = w1.shape
     l, s, r = w2.shape
-    d = dout_blk.permute(1, 0, 2)
+    d = dy.view(B, s, l).permute(2, 0, 1)
     dw2 = torch.bmm(d.transpose(-1, -2).contiguous(), out1)
     dt = torch.bmm(d.contiguous(), w2)
     dout1 = dt.transpose(0, 1).transpose(-1, -2).contiguous().reshape(B, k, q).transpose(0, 1).contiguous()
@@ -408,19 +423,20 @@ def butterfly_cpu_baseline(layer):
 
 
 def bench_butterfly(args, w):
-    from monarch_muon_amd import butterfly_blk_bwd_op, butterfly_blk_op
+    from monarch_muon_amd import butterfly_blk
     dev = torch.device("cuda", 0)
     tokens = args.tokens
     log(f"[bench] butterfly layer of {w.name}, {tokens} tokens, on {torch.cuda.get_device_name(dev)}")
-    layer = butterfly_layer(w, tokens, dev)
+    blocked = butterfly_layer(w, tokens, dev)
+    # the layer's own call: output and gradient in feature order
+    layer = [(name, x.requires_grad_(), w1.requires_grad_(), w2.requires_grad_(), d.transpose(1, 2).flatten(1))
+             for name, x, w1, w2, d in blocked]
     fwd_fl = sum(butterfly_flops(x, w1, w2) for _, x, w1, w2, _ in layer)
-    saved = {}
 
     def step():
-        for name, x, w1, w2, _ in layer:
-            saved[name] = butterfly_blk_op(x, w1, w2)[1]
-        for name, x, w1, w2, d in reversed(layer):
-            butterfly_blk_bwd_op(x, w1, w2, saved[name], d)
+        ys = [butterfly_blk(x, w1, w2) for _, x, w1, w2, _ in layer]
+        for (_, x, w1, w2, dy), y in zip(reversed(layer), reversed(ys)):
+            torch.autograd.grad(y, (x, w1, w2), dy)
 
     freeze_gc()
     for _ in range(args.warmup):
@@ -450,20 +466,25 @@ def bench_butterfly(args, w):
 
     per = {}
     fwd_ms = bwd_ms = ref_fwd_ms = ref_bwd_ms = 0.0
-    for name, x, w1, w2, d in layer:
+    for name, x, w1, w2, dy in layer:
         fl = butterfly_flops(x, w1, w2)
-        f = op_ms(lambda: butterfly_blk_op(x, w1, w2))
-        o1 = butterfly_blk_op(x, w1, w2)[1]
-        bw = op_ms(lambda: butterfly_blk_bwd_op(x, w1, w2, o1, d))
-        rf = op_ms(lambda: torch_reference_fwd(x, w1, w2))
-        rt = torch_reference_fwd(x, w1, w2)[1]
-        rb = op_ms(lambda: torch_reference_bwd(x, w1, w2, rt, d))
+        f = op_ms(lambda: butterfly_blk(x, w1, w2))
+        y = butterfly_blk(x, w1, w2)
+        bw = op_ms(lambda: torch.autograd.grad(y, (x, w1, w2), dy, retain_graph=True))
+        with torch.no_grad():
+            rf = op_ms(lambda: torch_reference_fwd(x, w1, w2))
+            rt = torch_reference_fwd(x, w1, w2)[1]
+            rb = op_ms(lambda: torch_reference_bwd(x, w1, w2, rt, dy))
         fwd_ms, bwd_ms, ref_fwd_ms, ref_bwd_ms = fwd_ms + f, bwd_ms + bw, ref_fwd_ms + rf, ref_bwd_ms + rb
         per[name] = {"w1": list(w1.shape), "w2": list(w2.shape), "fwd_ms": round(f, 4), "bwd_ms": round(bw, 4),
                      "fwd_tflops": round(fl / (f * 1e-3) / 1e12, 1), "bwd_tflops": round(2 * fl / (bw * 1e-3) / 1e12, 1),
                      "torch_fwd_ms": round(rf, 4), "torch_bwd_ms": round(rb, 4)}
-    # the dominant kernel: the forward product (two launches of butterfly_gemm<false, false, false>
-    # per forward call; the event pair around the call also holds the gap between them)
+    # the forward products (two launches per call: the riffled intermediate, then the output in feature
+    # order; the event pair around the call also holds the gap between them).  HBM bytes: of the 256-wide
+    # tiles, which every product of the 6.89B layer takes at 4096 tokens
+    fwd_kernels = [f"butterfly_gemm<Geo<2, 4, 4, 2, 4>, false, false, {out}>" for out in (0, 2)]
+    recorded = [hbm_traffic("butterfly-6.89b" if tokens == 4096 and w.name == "6.89b-nb4" else "-", k)
+                for k in fwd_kernels]
     fwd_avg_launch = fwd_ms / (2 * len(layer))
     achieved = fwd_fl / (fwd_ms * 1e-3) / 1e12
     total_fl = 3 * fwd_fl
@@ -478,21 +499,22 @@ def bench_butterfly(args, w):
         "median_event_ms": round(ev_ms, 4),
         "tflops": round(total_fl / (wall_ms * 1e-3) / 1e12, 1),
         "frac_peak": round(total_fl / (wall_ms * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4),
-        "roofline": {"bound": "mfma", "kernel": "butterfly_gemm<false, false, false>", "achieved": round(achieved, 1),
+        "roofline": {"bound": "mfma", "kernel": "the two forward products", "achieved": round(achieved, 1),
                      "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
-                     "traffic": hbm_traffic("butterfly-6.89b" if tokens == 4096 and w.name == "6.89b-nb4" else "-",
-                                            "butterfly_gemm<false, false, false>"),
+                     "traffic": sum(recorded) // 2 if None not in recorded else None,
                      "avg_launch_ms": round(fwd_avg_launch, 4),
                      "alg_flops_per_launch": fwd_fl / (2 * len(layer))},
         "forward_ms": round(fwd_ms, 4), "backward_ms": round(bwd_ms, 4),
         "torch_reference_ms": {"forward": round(ref_fwd_ms, 4), "backward": round(ref_bwd_ms, 4),
                                "total": round(ref_fwd_ms + ref_bwd_ms, 4),
-                               "note": "the reference's monarch_ops.py bmm + eager riffle path, same GPU, per-op events"},
+                               "note": "the reference's monarch_ops.py bmm + eager riffle path to the output in "
+                                       "feature order, same GPU, per-op events"},
         "projections": per,
     }
     if not args.no_cpu_baseline:
         log("[bench] CPU baseline (oracle on host cores, bounded sample)")
-        res["cpu_baseline"] = butterfly_cpu_baseline(layer)
+        res["cpu_baseline"] = butterfly_cpu_baseline([tuple(t.detach() if torch.is_tensor(t) else t for t in row)
+                                                      for row in blocked])
     print(json.dumps(res), flush=True)
 
 

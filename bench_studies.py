@@ -173,17 +173,16 @@ class PowerSampler:
 
 def stage_bytes(kind, gl):
     """Algorithmic HBM bytes of one launch of a Newton-Schulz stage over the
-    stored extents: bf16 X stacks (m_p x K rows x columns read, m_p x n_p
-    written), the upper 256 x 256 tiles of A and P, and for the last PX the
-    parameter block read and written instead of X'."""
+    stored extents: X stacks (m_p x K rows x columns read, m_p x n_p written), A
+    and P (bf16: their upper 256 x 256 tiles; fp32: whole), and for the last PX
+    the parameter block read and written instead of X'."""
     lay = gl.ws.layout
     N, mp, np_ = gl.nblocks, lay.mp, lay.np_
-    if gl.struct.ns_dtype == 0:   # fp32 kernels: 128 x 128 tiles, SYRK / POLY the upper ones only
-        kx = -(-lay.n // 32) * 32   # SYRK's K: n rounded up to the 32-deep K tiles
-        nt = mp // 128
-        up = (nt * (nt + 1) / 2) / (nt * nt)
-        full = {"syrk": mp * mp * kx * up, "poly": mp ** 3 * up, "px": mp * mp * np_, "px_apply": mp * mp * np_}
-        return 2.0 * full.get(kind, 0) * N
+    if gl.struct.ns_dtype == 0:
+        kx = -(-lay.n // 16) * 16   # SYRK's K: n rounded up to the 16-deep K steps
+        a, apply = 4 * mp * mp, 2 * gl.rows * gl.cols * (2 if gl.struct.param_dtype == 1 else 4)
+        return N * {"syrk": 4 * mp * kx + a, "poly": 2 * a, "px": a + 8 * mp * np_,
+                    "px_apply": a + 4 * mp * np_ + apply}[kind]
     side = [min(256, mp - i) for i in range(0, mp, 256)]   # the last tile may be partial
     up = mp * mp + sum(t * t for t in side)                  # bytes: half the square and half the diagonal tiles
     kx = -(-lay.n // 32) * 32
@@ -517,7 +516,7 @@ def traffic_summary(args):
     f, wr = counter_summary([fetch_csv]), counter_summary([write_csv])
     kernels = {}
     for k in f:
-        if k in wr and (k.startswith(("ns_", "pack", "adamw", "fp8_", "splitk")) or "butterfly" in k):
+        if k in wr and k.startswith(("ns_", "pack", "adamw", "fp8_", "splitk", "butterfly", "to_blocks")):
             b = f[k]["FETCH_SIZE"] * 1024 * fscale + wr[k]["WRITE_SIZE"] * 1024 * wscale
             kernels[k] = {"fetch_kib": f[k]["FETCH_SIZE"], "write_kib": wr[k]["WRITE_SIZE"], "bytes": b,
                           "read_bytes": f[k]["FETCH_SIZE"] * 1024 * fscale,
@@ -641,7 +640,7 @@ def stall_summary(args):
         wc = c.get("SQ_WAVE_CYCLES", 0.0)
         if wc <= 0 or "duration_ns" not in c:
             continue
-        if not (k.startswith(("ns_", "pack", "adamw", "fp8_", "splitk")) or "butterfly" in k):
+        if not k.startswith(("ns_", "pack", "adamw", "fp8_", "splitk", "butterfly", "to_blocks")):
             continue
         res[k] = {"dispatches": c["dispatches"], "avg_ms": round(c["duration_ns"] * 1e-6, 4),
                   "wait_any_frac": round(c["SQ_WAIT_ANY"] / wc, 3),
