@@ -33,13 +33,13 @@
 // backward splits dout's blocks in one pass (to_blocks_kernel).
 //
 // What bounds it, one 6.89B up-projection (4 x 1024 x 1024, 4 x 2752 x 1024) at 4096
-// tokens, forward + backward 563 -> 453 us with the output stored in feature order
-// (two strided copies of 63-72 us before, one pass of 27-35 now): the 256-wide products
-// spend 8 us of a 45 us round filling and draining the pipeline, and read and write LDS
-// as long as their MFMAs run.  At 4096 tokens of 4 x 512 x 512 the 128-wide tiles took
-// the six products from 157 to 121 us, at 1000 tokens of 2 x 256 x 256 the 64-wide ones
-// from 125 to 52.  Up to 64 tokens the forward's two products have a kernel of their
-// own (butterfly_few).
+// tokens, forward + backward 567 -> 457 us with the output stored in feature order
+// (two strided copies of 63-72 us before; now a pass of 33 over the gradient, and F2 takes
+// 118 us where the blocked store takes 96): the 256-wide products spend 8 us of a 45 us
+// round filling and draining the pipeline, and read and write LDS as long as their MFMAs
+// run.  At 4096 tokens of 4 x 512 x 512 the 128-wide tiles took the six products from 157
+// to 121 us, at 1000 tokens of 2 x 256 x 256 the 64-wide ones from 125 to 52.  Up to 64
+// tokens the forward's two products have a kernel of their own (butterfly_few).
 #include <algorithm>
 #include <atomic>
 
@@ -459,8 +459,13 @@ __device__ __forceinline__ void gemm_work(const GemmArgs& a, char* lds, int v) {
   if constexpr (OUT == OUT_FEATURES) {
     // bf16 straight from the accumulators: column j of batch g is feature j G + g of
     // the row, so a wave store puts 2 B at 32 places 2 G B apart in two rows; the
-    // other batches' tiles fill the rest of the lines in the same L2 (measured: as
-    // fast as the staged stores, and no interleaving pass follows)
+    // other batches' tiles fill the rest of the lines in the same L2: HBM writes are
+    // the output's bytes at 4 x 1024 columns, 2-12% more at 4 x 2752.  Slower than the
+    // staged stores of the blocked output (4096 tokens, us): 4 x 1024 x 1024 48.4
+    // against 42.9, 4 x 2752 x 1024 118 against 96, 4 x 512 x 512 18.3 against 16.6;
+    // for the same order the blocked output needs a copy, 63-72 for the second.  Part of
+    // the difference is reading: a group's G tiles share no operand, so 4 x 1024 x 1024
+    // fetches 101 MB where F1 of the same size fetches 50
     const GOut& c = a.c;
     const int lane = p.lane;
 #pragma unroll
@@ -697,9 +702,9 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* partial, int S
 // Feature order (B, s l) -> blocked rows (B, l, s): feature j l + b of a row is column j
 // of block b.  A thread reads 8 consecutive features (16 B) and writes 8 / l columns of
 // each block (one column of 8 of the 16 blocks), so a wave reads 1 KiB runs and writes
-// runs of 1 KiB / l per block.  HBM-bound: 4096 rows of 4 x 2752 take 27 us (90 MB, the
-// output stays in the Infinity Cache for the products that follow); a strided copy by
-// torch took 61.
+// runs of 1 KiB / l per block.  Bound by the copy rate: 4096 rows of 4 x 2752 are read
+// and written (90 MB each way, both counted at the L2) in 33 us, 5.4 TB/s, which is what a
+// large copy reaches; 4 x 1024 in 14.8 us, 4.5 TB/s.  A strided copy by torch took 61.
 template <int L>
 __global__ __launch_bounds__(256) void to_blocks_kernel(const uint16_t* src, uint16_t* dst, int64_t chunks, int s) {
   constexpr int U = 4;                        // chunks per thread
