@@ -947,6 +947,19 @@ constexpr int F_PAD = 128;             // padding granularity of the fp32 stacks
 // 480 tiles: SYRK 139 us with 64 x 64 tiles, 118 with 128 x 128; 44 blocks of 256 x
 // 256, 132 tiles: 12.4 against 16.3; 12 blocks of 256 x 688, 36 tiles: 16.1 against 29.7).
 constexpr int F32_FILL = 256;
+// Blocks go to XCDs whole, which keeps a block's operands, and what the stage before
+// wrote, in one L2 (48 blocks of 512 x 512: SYRK 48.9 us, 50.8 when every block is spread
+// over all XCDs; 64: 69.8 / 73.8), unless that fills some XCDs' 32 CUs more than once
+// while others idle: with one 2048 x 2048 block on one XCD SYRK takes 306 us, spread over
+// all 86; two 1024 x 1024 blocks 70 / 32, twelve (two on half of the XCDs, one on the
+// others) 123 / 87, twenty 162 / 142.  With a quarter of the slots idle spreading is as
+// fast or faster at every such size; from 512 on also with 15% (twenty 384 x 384: 15.9 /
+// 17.5, twenty 512 x 1376: 68.8 / 65.5; 9%, 44 blocks of 512 x 512: 48.3 / 50.6).  A step of
+// twelve 256 x 256 blocks, 20 tiles on the fullest XCD: 136 / 152.
+bool f32_spread(int blocks, int64_t tiles, int side) {
+  const int slots = (blocks + 7) / 8 * 8;
+  return slots / 8 * tiles > 32 && (4 * slots >= 5 * blocks || (side >= 512 && 20 * slots >= 23 * blocks));
+}
 
 template <int TW>
 struct F32Geo {
@@ -1102,7 +1115,7 @@ __device__ __forceinline__ void f32_update(typename TP::storage* prm, const NsAr
 }
 
 template <int STAGE, class TP, int TW>
-__global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(2))) void ns_f32(NsArgs a) {
+__global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(2))) void ns_f32(NsArgs a, int spread) {
   using G = F32Geo<TW>;
   constexpr int FT = G::FT, WT = G::WT;
   __shared__ __attribute__((aligned(1024))) char lds[G::LDS];
@@ -1111,7 +1124,12 @@ __global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(2))) void 
   const int nt = a.mp / FT, nc = a.np / FT;
   const int tiles = SYM ? nt * (nt + 1) / 2 : nt * nc;
   int b, t0;
-  if (!decode_tile(blockIdx.x, tiles, a.N, b, t0)) return;
+  if (spread) {
+    b = blockIdx.x / tiles;
+    t0 = blockIdx.x - b * tiles;
+  } else if (!decode_tile(blockIdx.x, tiles, a.N, b, t0)) {
+    return;
+  }
   int ti, tj;
   if (SYM) {
     f32_sym_tile(t0, nt, ti, tj);
@@ -1439,7 +1457,9 @@ void launch_f32_t(const NsArgs& a, hipStream_t s) {
     if (a.out) c.out = static_cast<float*>(a.out) + b0 * per_out;
     if (a.scale) c.scale = a.scale + b0;
     if (a.blocks) c.blocks = a.blocks + b0;
-    hipLaunchKernelGGL((ns_f32<STAGE, TP, TW>), dim3(unsigned(8 * ((c.N + 7) / 8) * tiles)), dim3(F_NT), 0, s, c);
+    const bool spread = f32_spread(c.N, tiles, a.mp);
+    const int slots = spread ? c.N : (c.N + 7) / 8 * 8;
+    hipLaunchKernelGGL((ns_f32<STAGE, TP, TW>), dim3(unsigned(slots * tiles)), dim3(F_NT), 0, s, c, int(spread));
   }
 }
 template <int STAGE, class TP>

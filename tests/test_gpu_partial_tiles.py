@@ -118,3 +118,15 @@ def test_fp32_with_singular_values_over_four_decades(sides):
     e = rel_fro(run_ns_only(g.to(DEV), None).double(), ns_fp64(g.double()))
     print("vs fp64", e.tolist())
     assert e.max() < 1e-5, e
+
+
+@pytest.mark.parametrize("sides", [(256, 256), (512, 640), (1032, 520)], ids=ids)
+def test_fp32_blocks_do_not_depend_on_their_number(sides):
+    """One to 24 blocks: dealt to the XCDs whole (8, 16, 24) or spread over them, in 64- and in 128-wide tiles; a
+    block's result is the same, bit for bit."""
+    print("number of blocks", sides, flush=True)
+    g = (torch.randn((24, *sides), generator=torch.Generator().manual_seed(9)) * 1e-3).to(DEV)
+    want = run_ns_only(g, None)
+    assert rel_fro(want[:2].double(), ns_fp64(g[:2].cpu().double())).max() < 1e-5
+    for n in (1, 2, 3, 5, 8, 12, 16, 20, 23):
+        assert torch.equal(run_ns_only(g[:n], None), want[:n]), n
