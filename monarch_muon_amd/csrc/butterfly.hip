@@ -847,6 +847,18 @@ void launch_gemm_t(const GemmArgs& a, hipStream_t s) {
   else launch_gemm_g<G64, AT, BT, OUT>(a, s);
 }
 
+// Products that take butterfly_few.  It reads all tokens once per 16 features, so with
+// many features the 64-wide tiles, once they fill the chip, overtake it: at 512 of them from
+// 17 tokens on (16 x 2048 x 2048, forward us, few / tiles: 16 tokens 58 / 60, 17 68 / 61, 64
+// 124 / 65), at 256 between 33 and 64 (16 x 1024 x 1024: 32 tokens 22.7 / 25.0, 33 25.7 /
+// 24.9, 64 33 / 27; 8 x 2048 x 2048 35.9 / 35.3, 36.4 / 35.5, 46 / 37; 4 x 4096 x 4096 70 /
+// 94, 78 / 93, 103 / 100), below not up to 64 (8 x 1024 x 1024, 128 tiles: 19.0 / 22.0).
+bool few_tokens(const GemmArgs& a) {
+  if (a.M > FEW_TOKENS) return false;
+  const int64_t tiles = int64_t(a.G) * cdiv(a.N, 64);
+  return a.M <= 16 || tiles < 256 || tiles * cdiv(a.M, 16) <= 512;
+}
+
 template <int NT, int RING, bool FEATURES>
 void launch_few_t(const GemmArgs& a, hipStream_t s) {
   constexpr int LW = 4, U = 4;
@@ -921,14 +933,14 @@ int launch_butterfly_fwd(const mmuon_butterfly_args& x, bool features, hipStream
   f1.c = make_out(x.out1, ql * 2, int64_t(d.q) * 2, UNSEG, 0, d.log2l, d.B * d.q * 2);
   // (a 64-wide tile of 16 planes would write runs shorter than 16 B)
   set_geometry(f1, int(d.B), d.q, d.p, d.nb, gemm_plan(d.B, d.q, d.nb, d.p, false, d.nb > 8));
-  const bool few = d.B <= FEW_TOKENS;
-  if (few) launch_few<false>(f1, st);
+  if (few_tokens(f1)) launch_few<false>(f1, st);
   else launch_gemm_t<false, false, OUT_TILE>(f1, st);
   GemmArgs f2{};  // out[:, ll] = t[ll] . w2[ll]^T
   f2.a = make_op(x.out1, d.B * d.q * 2, int64_t(d.q) * 2, 2, int(d.B));
   f2.b = make_op(x.w2, int64_t(d.s) * d.q * 2, int64_t(d.q) * 2, 2, d.s);
   f2.c = make_out(x.out, int64_t(d.s) * 2, int64_t(d.nb) * d.s * 2);
   set_geometry(f2, int(d.B), d.s, d.q, d.nb, gemm_plan(d.B, d.s, d.nb, d.q, false));
+  const bool few = few_tokens(f2);
   if (few && features && d.nb > 1) launch_few<true>(f2, st);
   else if (few) launch_few<false>(f2, st);
   else if (features && d.nb > 1) launch_gemm_t<false, false, OUT_FEATURES>(f2, st);

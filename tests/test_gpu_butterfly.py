@@ -152,6 +152,23 @@ def test_rows_do_not_depend_on_the_token_count(dims):
         assert torch.equal(butterfly_blk_bwd_op(x[:n], w1, w2, o1, dout[:n])[0], dx[:n]), n
 
 
+@pytest.mark.parametrize("dims", [(16, 2048, 264, 136), (16, 1024, 520, 1032), (4, 4096, 72, 4104)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_few_tokens_of_many_features(dims):
+    """Where the few-token kernel gives way to the tiles by the number of features, one product or both, on both sides
+    of each token count: the rows of a call of 300 tokens, which are within the pair's bar."""
+    print("many features", dims, flush=True)
+    x, w1, w2, _ = gpu(*make(300, *dims, seed=13))
+    out, out1 = butterfly_blk_op(x, w1, w2)
+    y = butterfly_blk(x, w1, w2)
+    ref_out, ref_out1 = bf.butterfly_fwd(x, w1, w2)
+    assert rel(out, ref_out) <= TOL and rel(out1, ref_out1) <= TOL
+    for n in (1, 16, 17, 32, 33, 48, 49, 64, 65):
+        o, o1 = butterfly_blk_op(x[:n], w1, w2)
+        assert torch.equal(o1, out1[:, :n]) and torch.equal(o, out[:n]), n
+        assert torch.equal(butterfly_blk(x[:n], w1, w2), y[:n]), n
+
+
 @pytest.mark.parametrize("how", ["compile", "saved_hooks", "expanded_grad", "second_order"])
 def test_layer_operator_under_torch(how):
     """The native operator traced by torch.compile, with saved-tensor hooks and with a gradient that is no dense
