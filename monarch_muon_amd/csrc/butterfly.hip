@@ -789,6 +789,10 @@ enum { T256 = 0, T128 = 1, T64 = 2 };
 // 1024 44 / 58 / 96; 1000 tokens of 2 x 256 x 256 14.4 / 8.8 / 7.1; 8 tokens of 4 x 1024
 // x 1024 26 / 14 / 12.  (256 x 128 tiles, two workgroups per CU, were slower than 256 x
 // 256 wherever those fill the chip: 54 against 46 us on 16384 tokens of 2 x 512 x 1368.)
+// A last round of few 256-wide tiles runs at their unloaded rate: 288 of them (2049 tokens
+// of 4 x 2048 x 2048) 100 us a product against 109 in 128-wide ones, with K = 2464 (8 x 1024)
+// 173 / 194 both products, 576 (9000 tokens of 8 x 512 x 512) 65 / 68.  Counted for the
+// products whose sums do not depend on the choice; a weight gradient's splits stay.
 struct GemmPlan {
   int tile, S;
 };
@@ -796,8 +800,10 @@ int64_t gemm_cost(int tile, int64_t M, int64_t N, int64_t G, int64_t K, int64_t 
   const int64_t side = tile == T256 ? 256 : tile == T128 ? 128 : 64;
   const int64_t tiles = G * S * ((M + side - 1) / side) * ((N + side - 1) / side);
   const int64_t rounds = (tiles + 255) / 256, k = (K + S - 1) / S;
+  const auto one_round = [k](int64_t n) { return n > 0 ? 8000 + k * (22 + 14 * n / 256) : 0; };
   int64_t t;
-  if (tile == T256) t = rounds * (8000 + k * (22 + 14 * std::min<int64_t>(tiles, 256) / 256));
+  if (tile == T256 && !wgrad) t = tiles / 256 * one_round(256) + one_round(tiles % 256);
+  else if (tile == T256) t = rounds * (8000 + k * (22 + 14 * std::min<int64_t>(tiles, 256) / 256));
   else if (tile == T128) t = 4000 + rounds * (1000 + k * (wgrad ? 14 : rounds == 1 ? 9 : rounds == 2 ? 11 : 14));
   else t = 4700 + std::max<int64_t>(tiles, 256) * (300 + k * 13 / 2) / 256;
   // splits: the partials' write and read, and the reduction's launch
