@@ -43,10 +43,11 @@ static_assert(LDS_ELEMS >= BN * 256, "the staged tile fits in the ring");
 // workgroup resident), so virtual tile w runs on XCD w % 8.  Map w to
 // (block, tile) so that every tile of one block lands on the same XCD (and its
 // L2), and the tiles of a block run in the same round: they start together and
-// stream the block's panels in step, which the L2 serves.
-__device__ __forceinline__ bool decode_tile(int w, int tiles, int N, int& b, int& t) {
-  const int xcd = w & 7, local = w >> 3;
-  b = xcd + 8 * (local / tiles);
+// stream the block's panels in step, which the L2 serves.  spread: block by block, the
+// tiles of each dealt to all XCDs.
+__device__ __forceinline__ bool decode_tile(int w, int tiles, int N, int& b, int& t, int spread = 0) {
+  const int xcd = w & 7, local = spread ? w : w >> 3;
+  b = spread ? local / tiles : xcd + 8 * (local / tiles);
   t = local % tiles;
   return b < N;
 }

@@ -956,9 +956,12 @@ constexpr int F32_FILL = 256;
 // fast or faster at every such size; from 512 on also with 15% (twenty 384 x 384: 15.9 /
 // 17.5, twenty 512 x 1376: 68.8 / 65.5; 9%, 44 blocks of 512 x 512: 48.3 / 50.6).  A step of
 // twelve 256 x 256 blocks, 20 tiles on the fullest XCD: 136 / 152.
-bool f32_spread(int blocks, int64_t tiles, int side) {
-  const int slots = (blocks + 7) / 8 * 8;
-  return slots / 8 * tiles > 32 && (4 * slots >= 5 * blocks || (side >= 512 && 20 * slots >= 23 * blocks));
+// The same for every stage of a chain, from its SYRK's 64-wide tiles (PX of the twelve
+// 256 x 688 blocks spread between stages that are not: the toy model's step 797 / 804 us).
+bool f32_spread(int blocks, int side) {
+  const int slots = (blocks + 7) / 8 * 8, nt = side / 64;
+  return slots / 8 * int64_t(nt * (nt + 1) / 2) > 32 &&
+         (4 * slots >= 5 * blocks || (side >= 512 && 20 * slots >= 23 * blocks));
 }
 
 template <int TW>
@@ -1124,12 +1127,7 @@ __global__ __launch_bounds__(F_NT) __attribute__((amdgpu_waves_per_eu(2))) void 
   const int nt = a.mp / FT, nc = a.np / FT;
   const int tiles = SYM ? nt * (nt + 1) / 2 : nt * nc;
   int b, t0;
-  if (spread) {
-    b = blockIdx.x / tiles;
-    t0 = blockIdx.x - b * tiles;
-  } else if (!decode_tile(blockIdx.x, tiles, a.N, b, t0)) {
-    return;
-  }
+  if (!decode_tile(blockIdx.x, tiles, a.N, b, t0, spread)) return;
   int ti, tj;
   if (SYM) {
     f32_sym_tile(t0, nt, ti, tj);
@@ -1457,7 +1455,7 @@ void launch_f32_t(const NsArgs& a, hipStream_t s) {
     if (a.out) c.out = static_cast<float*>(a.out) + b0 * per_out;
     if (a.scale) c.scale = a.scale + b0;
     if (a.blocks) c.blocks = a.blocks + b0;
-    const bool spread = f32_spread(c.N, tiles, a.mp);
+    const bool spread = f32_spread(c.N, a.mp);
     const int slots = spread ? c.N : (c.N + 7) / 8 * 8;
     hipLaunchKernelGGL((ns_f32<STAGE, TP, TW>), dim3(unsigned(slots * tiles)), dim3(F_NT), 0, s, c, int(spread));
   }
